@@ -433,6 +433,283 @@ __global__ __launch_bounds__(256) void recurrent_fwd_kernel(RecurrentParams p)
     }
 }
 
+// Sum over the 16 row groups of a lane's column.  The row group sits in lane
+// bits 0, 1, 4, 5: two quad permutations and the two row swaps, each an exact
+// butterfly (both partners add the same two values, so every row group ends
+// with the same bits) on the VALU -- a shuffle through the LDS pipe would put
+// four round trips of about 50 cycles on the token chain.
+__device__ __forceinline__ float swap_add16(float x)
+{
+    const unsigned u = __float_as_uint(x);
+    const auto s = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+    return __uint_as_float(s[0]) + __uint_as_float(s[1]);
+}
+
+__device__ __forceinline__ float swap_add32(float x)
+{
+    const unsigned u = __float_as_uint(x);
+    const auto s = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+    return __uint_as_float(s[0]) + __uint_as_float(s[1]);
+}
+
+template <int CTRL>
+__device__ __forceinline__ float dpp_add(float x)
+{
+    return x + __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(x), CTRL, 0xf, 0xf, true));
+}
+
+__device__ __forceinline__ float rowgroup_sum(float x)
+{
+    x = dpp_add<0xb1>(x);  // quad_perm [1, 0, 3, 2]
+    x = dpp_add<0x4e>(x);  // quad_perm [2, 3, 0, 1]
+    return swap_add32(swap_add16(x));
+}
+
+// Sum over all 64 lanes, the same bits in every lane.
+__device__ __forceinline__ float wave_sum_dpp(float x)
+{
+    x = dpp_add<0xb1>(x);
+    x = dpp_add<0x4e>(x);
+    x = dpp_add<0x141>(x);  // row_half_mirror: the quads hold equal values
+    x = dpp_add<0x140>(x);  // row_mirror
+    return swap_add32(swap_add16(x));
+}
+
+// NC consecutive state columns (state rows are 16-byte aligned, V a multiple of 4).
+template <int NC>
+struct alignas(4 * NC) StateCols {
+    float e[NC];
+};
+
+template <int NC>
+__device__ __forceinline__ void put_cols(float *dst, const float (&x)[NC])
+{
+    StateCols<NC> y;
+#pragma unroll
+    for (int c = 0; c < NC; ++c) y.e[c] = x[c];
+    *reinterpret_cast<StateCols<NC> *>(dst) = y;
+}
+
+// Token-serial forward of sequences of several tokens.
+//
+// What bounds it is the token chain (a token's update needs the sum over all
+// K rows of the state before it), so the kernel shortens the chain and takes
+// everything else off it:
+//   - Columns of the state are independent: a workgroup owns 16 * NC of them
+//     (a wave 4 * NC), a (sequence, head) spans V / (16 NC) workgroups.  NC is
+//     the widest that still gives every CU a workgroup (launch_seq).
+//   - Lane (rg, cl) holds rows rg + 16 i of NC columns, so a sum over K is
+//     NR = KP/16 chained FMAs and four VALU butterfly steps, no LDS, no barrier.
+//   - A tile of TT tokens is prepared at once (norms, decays, b*k), one wave a
+//     token, and left in LDS as float4 (a, a e, a q, k) a row: one 16-byte read
+//     gives a lane all a row needs, the next token's rows are read while the
+//     current one's chain runs.  r = S^T (a e) and the o partial S^T (a q) are
+//     taken from the state before its decay, which leaves one FMA per row after
+//     the sum:  S <- a S + k u.
+//   - The next tile's inputs are requested before the tile's token loop.
+// Two prompts of 48 tokens, 16 heads, d = 128: 26 us (kernel alone), where one
+// workgroup per head with three barriers a token took 152 us; 2048 tokens of 16
+// heads 0.90 ms, before 6.83.
+template <typename TI, typename TG, int KP, int NC>
+__global__ __launch_bounds__(256) void recurrent_seq_kernel(RecurrentParams p)
+{
+    constexpr int RG = 16, NR = KP / RG, CPL = KP / kWave;
+    constexpr int TT = KP <= 128 ? 16 : 8, TW = TT / 4;  // tokens of a tile, of a wave
+    constexpr int CB = 16 * NC;                          // columns of the workgroup
+    constexpr int VE = TT * CB / 256;                    // v / w elements of a thread
+    static_assert(KP % kWave == 0 && TT * CB % 256 == 0, "seq mapping");
+
+    const int K = p.K, V = p.V;
+    const int n = blockIdx.x / p.HV, hv = blockIdx.x % p.HV;
+    const int h = hv / (p.HV / p.H);
+    int64_t bos, len;
+    if (p.cu_seqlens) {
+        bos = p.cu_seqlens[n];
+        len = p.cu_seqlens[n + 1] - bos;
+    } else {
+        bos = static_cast<int64_t>(n) * p.T;
+        len = p.T;
+    }
+
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), wid = tid / kWave;
+    const int rg = (lane & 3) | ((lane >> 4) << 2), cl = (lane >> 2) & 3;
+    const int c0 = blockIdx.y * CB, lc = (wid * 4 + cl) * NC, col = c0 + lc;
+    const bool col_ok = col < V;  // NC divides 4 and V is a multiple of 4
+
+    __shared__ float4 s_tok[TT][KP];
+    __shared__ float s_vw[TT][CB], s_o[TT][CB], s_kq[TT];
+
+    const TI *q = static_cast<const TI *>(p.q), *k = static_cast<const TI *>(p.k);
+    const TI *v = static_cast<const TI *>(p.v), *w = static_cast<const TI *>(p.w);
+    const TI *b = static_cast<const TI *>(p.b);
+    const TG *g = static_cast<const TG *>(p.g);
+    TI *o = static_cast<TI *>(p.o);
+    const bool l2 = (p.flags & GDN2_FLAG_L2NORM_QK) != 0;
+    const bool gate = (p.flags & GDN2_FLAG_GATE_IN_KERNEL) != 0;
+    const int use_lb = (p.flags & GDN2_FLAG_LOWER_BOUND) != 0;
+    const bool sig_bw = (p.flags & GDN2_FLAG_SIGMOID_BW) != 0;
+    const bool per_token = p.state_indices != nullptr;
+
+    float st[NR][NC];
+    const float *h0row = initial_row(p, n, hv);
+#pragma unroll
+    for (int i = 0; i < NR; ++i) {
+        const int r = rg + i * RG;
+        StateCols<NC> x = {};
+        if (h0row && col_ok && r < K)
+            x = *reinterpret_cast<const StateCols<NC> *>(h0row + static_cast<int64_t>(r) * V + col);
+#pragma unroll
+        for (int c = 0; c < NC; ++c) st[i][c] = x.e[c];
+    }
+    float a_log = 0.0f, dtb[CPL];
+    if (gate) a_log = p.A_log[h];
+#pragma unroll
+    for (int j = 0; j < CPL; ++j) {
+        const int c = lane + kWave * j;
+        dtb[j] = gate && p.dt_bias && c < K ? p.dt_bias[h * K + c] : 0.0f;
+    }
+
+    // Wave wid prepares tokens wid + 4 i of a tile, thread tid elements
+    // tid + 256 i of the v / w tile.  Positions past the end read the last token.
+    float rq[TW][CPL], rk[TW][CPL], rb[TW][CPL], rgv[TW][CPL], rv[VE], rw[VE];
+    auto request = [&](int64_t t0) {
+#pragma unroll
+        for (int i = 0; i < TW; ++i) {
+            const int64_t t = t0 + wid + 4 * i, tok = bos + (t < len ? t : len - 1);
+#pragma unroll
+            for (int j = 0; j < CPL; ++j) {
+                const int c = lane + kWave * j, cc = c < K ? c : K - 1;
+                rq[i][j] = io<TI>::ld(q, (tok * p.H + h) * K + cc);
+                rk[i][j] = io<TI>::ld(k, (tok * p.H + h) * K + cc);
+                rb[i][j] = io<TI>::ld(b, (tok * p.HV + hv) * K + cc);
+                rgv[i][j] = io<TG>::ld(g, (tok * p.HV + hv) * K + cc);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < VE; ++i) {
+            const int e = tid + 256 * i, cv = c0 + e % CB;
+            const int64_t t = t0 + e / CB, tok = bos + (t < len ? t : len - 1);
+            const int64_t at = (tok * p.HV + hv) * V + (cv < V ? cv : V - 1);
+            rv[i] = io<TI>::ld(v, at);
+            rw[i] = io<TI>::ld(w, at);
+        }
+    };
+
+    if (len > 0) request(0);
+    for (int64_t t0 = 0; t0 < len; t0 += TT) {
+        const int nt = len - t0 < TT ? static_cast<int>(len - t0) : TT;
+#pragma unroll
+        for (int i = 0; i < TW; ++i) {
+            const int t = wid + 4 * i;
+            if (t >= nt) break;  // uniform over the wave
+            float qq = 0.f, kk = 0.f, qk = 0.f;
+#pragma unroll
+            for (int j = 0; j < CPL; ++j) {
+                if (lane + kWave * j >= K) rq[i][j] = rk[i][j] = 0.0f;
+                qq += rq[i][j] * rq[i][j];
+                kk += rk[i][j] * rk[i][j];
+                qk += rq[i][j] * rk[i][j];
+            }
+            qq = wave_sum_dpp(qq);
+            kk = wave_sum_dpp(kk);
+            qk = wave_sum_dpp(qk);
+            const float invq = l2 ? 1.0f / fmaxf(sqrtf(qq), 1e-6f) : 1.0f;
+            const float invk = l2 ? 1.0f / fmaxf(sqrtf(kk), 1e-6f) : 1.0f;
+#pragma unroll
+            for (int j = 0; j < CPL; ++j) {
+                const float bv = sig_bw ? sigmoid_f(rb[i][j]) : rb[i][j];
+                const float gk = gate ? gate_activation(rgv[i][j], a_log, dtb[j], use_lb, p.lower_bound) : rgv[i][j];
+                const float a = expf(gk), kn = rk[i][j] * invk;
+                const float4 x = make_float4(a, a * (bv * kn), a * (rq[i][j] * invq * p.scale), kn);
+                s_tok[t][lane + kWave * j] =
+                    lane + kWave * j < K ? x : make_float4(0.f, 0.f, 0.f, 0.f);
+            }
+            if (lane == 0) s_kq[t] = qk * invq * invk * p.scale;
+        }
+#pragma unroll
+        for (int i = 0; i < VE; ++i) {
+            const int e = tid + 256 * i;
+            const float wv = sig_bw ? sigmoid_f(rw[i]) : rw[i];
+            s_vw[e / CB][e % CB] = wv * rv[i];
+        }
+        request(t0 + TT);
+        __syncthreads();
+
+        float4 x[NR];
+        float vw[NC], kq = s_kq[0];
+#pragma unroll
+        for (int i = 0; i < NR; ++i) x[i] = s_tok[0][rg + i * RG];
+#pragma unroll
+        for (int c = 0; c < NC; ++c) vw[c] = s_vw[0][lc + c];
+        for (int t = 0; t < nt; ++t) {
+            const int tn = t + 1 < TT ? t + 1 : t;
+            float r[NC], po[NC];
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+                // Two chains over the rows: half the FMA latency before the sum.
+                float r0 = st[0][c] * x[0].y, r1 = st[1][c] * x[1].y;
+                float p0 = st[0][c] * x[0].z, p1 = st[1][c] * x[1].z;
+#pragma unroll
+                for (int i = 2; i < NR; i += 2) {
+                    r0 = fmaf(st[i][c], x[i].y, r0);
+                    r1 = fmaf(st[i + 1][c], x[i + 1].y, r1);
+                    p0 = fmaf(st[i][c], x[i].z, p0);
+                    p1 = fmaf(st[i + 1][c], x[i + 1].z, p1);
+                }
+                r[c] = r0 + r1;
+                po[c] = p0 + p1;
+            }
+            float4 xn[NR];
+            float vn[NC];
+            const float kqn = s_kq[tn];
+#pragma unroll
+            for (int i = 0; i < NR; ++i) xn[i] = s_tok[tn][rg + i * RG];
+#pragma unroll
+            for (int c = 0; c < NC; ++c) vn[c] = s_vw[tn][lc + c];
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+                const float u = vw[c] - rowgroup_sum(r[c]);
+#pragma unroll
+                for (int i = 0; i < NR; ++i) st[i][c] = fmaf(st[i][c], x[i].x, x[i].w * u);
+                const float oc = fmaf(u, kq, rowgroup_sum(po[c]));
+                if (rg == 0) s_o[t][lc + c] = oc;
+            }
+            if (per_token) {
+                float *dst = store_row(p, n, hv, t0 + t, bos + t0 + t);
+                if (dst && col_ok) {
+#pragma unroll
+                    for (int i = 0; i < NR; ++i) {
+                        const int row = rg + i * RG;
+                        if (row < K) put_cols(dst + static_cast<int64_t>(row) * V + col, st[i]);
+                    }
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < NR; ++i) x[i] = xn[i];
+#pragma unroll
+            for (int c = 0; c < NC; ++c) vw[c] = vn[c];
+            kq = kqn;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < VE; ++i) {
+            const int e = tid + 256 * i, t = e / CB, cv = c0 + e % CB;
+            if (t < nt && cv < V) io<TI>::st(o, ((bos + t0 + t) * p.HV + hv) * V + cv, s_o[t][e % CB]);
+        }
+    }
+
+    if (!per_token) {
+        float *dst = store_row(p, n, hv, len - 1, bos + len - 1);
+        if (dst && col_ok) {
+#pragma unroll
+            for (int i = 0; i < NR; ++i) {
+                const int row = rg + i * RG;
+                if (row < K) put_cols(dst + static_cast<int64_t>(row) * V + col, st[i]);
+            }
+        }
+    }
+}
+
 // Decode step (T = 1, no cu_seqlens) specialised for d_k = d_v = 128.
 // Same arithmetic and thread mapping as recurrent_fwd_kernel, but each
 // workgroup walks two consecutive (sequence, value head) slabs and issues the
@@ -1122,6 +1399,24 @@ static hipError_t launch_nr(const RecurrentParams &p, int N, hipStream_t stream)
     return hipGetLastError();
 }
 
+template <typename TI, typename TG, int KP>
+static hipError_t launch_seq(const RecurrentParams &p, int N, hipStream_t stream)
+{
+    // Columns per workgroup: 16 * NC, the widest whose grid still covers the
+    // 256 CUs; per-token state stores take 64-column workgroups, whose lanes
+    // store 16 bytes.
+    const int64_t heads = static_cast<int64_t>(N) * p.HV;
+    auto grid = [&](int nc) { return dim3(N * p.HV, (p.V + 16 * nc - 1) / (16 * nc)); };
+    auto covers = [&](int nc) { return heads * grid(nc).y >= 256; };
+    if (p.state_indices || covers(4))
+        hipLaunchKernelGGL((recurrent_seq_kernel<TI, TG, KP, 4>), grid(4), dim3(256), 0, stream, p);
+    else if (KP > 128 || covers(2))  // an 8-token tile of 16 columns does not fill 256 threads
+        hipLaunchKernelGGL((recurrent_seq_kernel<TI, TG, KP, 2>), grid(2), dim3(256), 0, stream, p);
+    else if constexpr (KP <= 128)
+        hipLaunchKernelGGL((recurrent_seq_kernel<TI, TG, KP, 1>), grid(1), dim3(256), 0, stream, p);
+    return hipGetLastError();
+}
+
 template <typename TI, typename TG>
 static hipError_t launch_tpr(const RecurrentParams &p, int N, hipStream_t stream)
 {
@@ -1138,6 +1433,19 @@ static hipError_t launch_tpr(const RecurrentParams &p, int N, hipStream_t stream
         else
             hipLaunchKernelGGL((decode_step_kernel<TI, TG, false>), grid, dim3(256), 0, stream, p, nslabs);
         return hipGetLastError();
+    }
+    // Sequences of several tokens (two on average when packed; their lengths
+    // are on the device).  Two or three tokens of very many heads are bound by
+    // the state's bytes, which the whole-row accesses of recurrent_fwd_kernel
+    // move faster: 64 x 2 tokens of 16 heads (d = 128) 37.5 us there, 42.0 us
+    // here; 1 x 2 tokens 11.9 and 6.0 us, 64 x 4 tokens from a pool 77.9 and 78.0,
+    // 64 x 16 tokens 137 and 100.
+    const int64_t heads = static_cast<int64_t>(N) * p.HV;
+    const bool several = p.T > 1 && (!p.cu_seqlens || p.T >= 2 * static_cast<int64_t>(N));
+    if (!trans && several && !(!p.cu_seqlens && p.T < 4 && heads >= 512)) {
+        if (p.K <= 64) return launch_seq<TI, TG, 64>(p, N, stream);
+        if (p.K <= 128) return launch_seq<TI, TG, 128>(p, N, stream);
+        return launch_seq<TI, TG, 256>(p, N, stream);
     }
     // Narrowest row that still covers V with float4 lanes, capped at 128 columns.
     if (p.V <= 16) return launch_nr<TI, TG, 4>(p, N, stream);
