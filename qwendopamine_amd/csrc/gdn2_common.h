@@ -80,6 +80,43 @@ __device__ __forceinline__ float wave_sum(float x)
     return x;
 }
 
+// Sum over k < nparts of part[k * E + e] for the workgroup's 64 elements e (one per
+// lane, every wave the same 64; e clamped to a valid element by the caller),
+// in a fixed order: wave w of NW takes the parts k = w mod NW with U requests
+// in flight, the waves' sums meet in LDS.  Valid in wave 0.  What bounds it is the
+// chain of waits, not the bytes: few elements mean few workgroups, so each
+// takes sixteen waves (the kernels that call it give the times).
+template <int NW, int U>
+__device__ __forceinline__ float sum_parts(const float *part, int64_t nparts, int64_t E, int64_t e,
+                                           float (*s_sum)[64])
+{
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    float a[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) a[u] = 0.0f;
+    int64_t k = wv;
+    for (; k + (U - 1) * NW < nparts; k += U * NW) {
+        float x[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) x[u] = part[(k + u * NW) * E + e];
+#pragma unroll
+        for (int u = 0; u < U; ++u) a[u] += x[u];
+    }
+    for (; k < nparts; k += NW) a[0] += part[k * E + e];
+#pragma unroll
+    for (int w = U / 2; w > 0; w >>= 1)
+#pragma unroll
+        for (int u = 0; u < w; ++u) a[u] += a[u + w];
+    s_sum[wv][lane] = a[0];
+    __syncthreads();
+    float s = 0.0f;
+    if (wv == 0) {
+#pragma unroll
+        for (int w = 0; w < NW; ++w) s += s_sum[w][lane];
+    }
+    return s;
+}
+
 // torch.nn.functional.softplus with its default threshold of 20, from the
 // hardware exp2 / log2 instead of the library expf / log1pf (which cost about
 // as much as the rest of the prologue):  max(x, 0) + log1p(e^-|x|), with

@@ -14,7 +14,7 @@
 //  * partial_reduce_kernel -- sums the partials over tiles / waves in a fixed
 //    order (deterministic) and writes the weight-shaped gradients.
 //
-// All three are HBM-bound elementwise / reduction passes.
+// All are elementwise / reduction passes.
 
 #include <type_traits>
 
@@ -25,10 +25,24 @@ namespace gdn2 {
 
 namespace {
 
+// sigmoid(x): 16-bit tensors take the hardware exp2 and reciprocal (1 ulp each in
+// fp32) that their forward took, float32 ones the library's exponential and an IEEE
+// divide.  The convolution's backward, bound by its instructions, went from 23.5 to
+// 18.8 us at 8192 tokens x 1024 channels in bf16 with them.
+template <typename T>
+__device__ __forceinline__ float sigmoid_of(float x)
+{
+    if constexpr (sizeof(T) == 2)
+        return sigmoid_f(x);
+    else
+        return 1.0f / (1.0f + expf(-x));
+}
+
 // silu'(x) = sigmoid(x) (1 + x (1 - sigmoid(x))), torch's formula.
+template <typename T>
 __device__ __forceinline__ float silu_grad(float x)
 {
-    const float s = 1.0f / (1.0f + expf(-x));
+    const float s = sigmoid_of<T>(x);
     return s * (1.0f + x * (1.0f - s));
 }
 
@@ -81,7 +95,7 @@ __global__ __launch_bounds__(256) void short_conv_bwd_kernel(ConvBwdParams p)
 #pragma unroll
         for (int j = 0; j < W; ++j) acc = fmaf(wt[j], xin[r + j], acc);
         const float pre = round_to<T>(acc + bias);  // the forward's rounded conv output
-        const float g = p.silu ? round_to<T>(gin[r] * silu_grad(pre)) : gin[r];
+        const float g = p.silu ? round_to<T>(gin[r] * silu_grad<T>(pre)) : gin[r];
         dpre[r] = t0 + r < p.T ? g : 0.0f;
     }
     float dw[W], db = 0.0f;
@@ -189,30 +203,110 @@ __global__ __launch_bounds__(256) void gated_rmsnorm_bwd_kernel(NormBwdParams p)
         p.part[static_cast<int64_t>(blockIdx.x) * N + c] = (s_acc[0][c] + s_acc[1][c]) + (s_acc[2][c] + s_acc[3][c]);
 }
 
-// out[e] = sum over k < nparts of part[k * E + e], e < E, in a fixed order
-// (deterministic): workgroup b takes 64 consecutive e, its four waves the
-// parts k = w mod 4 with four accumulators each, combined in LDS.  Written in
-// TO.  With W > 0, elements e = j * D + d of [W + 1][D] partials go to a
-// [D][W] weight (j < W) and a [D] bias (j == W).
-template <typename TO>
-__global__ __launch_bounds__(256) void partial_reduce_kernel(const float *part, int64_t nparts, int64_t E,
-                                                             void *out, void *out_bias, int D, int W)
+// The same gradients with 16-byte accesses: LPR lanes a row, EPV values a lane
+// (N = LPR * EPV), so a wave takes 64 / LPR rows at once, RPT of them in flight
+// per lane, and a row's two sums are log2(LPR) shuffles.  For rows of LPR (a power of
+// two, 8 to 32 in 16 bits, to 64 in 32) whole 16-byte pieces; the others stay on the kernel above.
+// HBM-bound by its bytes (x, z, dy, dx, dz: 10 a value in bf16); one 2-byte value a lane
+// left it bound by shuffles and instructions: 32.6 us at 131072 rows of 64 in
+// bf16, now 17.7 (84 MB: 4.7 TB/s).
+template <typename T, typename TW, int LPR>
+__global__ __launch_bounds__(256) void gated_rmsnorm_bwd_vec_kernel(NormBwdParams p)
 {
-    __shared__ float s_sum[4][64];
+    constexpr int EPV = 16 / static_cast<int>(sizeof(T)), N = LPR * EPV;
+    constexpr int RPW = 64 / LPR, RPT = 2, STEP = 4 * RPW * RPT;
+    __shared__ float s_acc[4][N];
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int64_t e = static_cast<int64_t>(blockIdx.x) * 64 + lane;
-    const int64_t ec = e < E ? e : E - 1;
-    float a[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    int64_t k = wv;
-    for (; k + 12 < nparts; k += 16) {
+    const int sub = lane / LPR, c0 = EPV * (lane % LPR);
+    const T *x = static_cast<const T *>(p.x);
+    const T *z = static_cast<const T *>(p.z);
+    const T *dy = static_cast<const T *>(p.dy);
+    T *dx = static_cast<T *>(p.dx);
+    T *dz = static_cast<T *>(p.dz);
+    float w[EPV], acc[EPV];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) a[u] += part[(k + 4 * u) * E + ec];
+    for (int i = 0; i < EPV; ++i) {
+        w[i] = io<TW>::ld(static_cast<const TW *>(p.weight), c0 + i);
+        acc[i] = 0.0f;
     }
-    for (; k < nparts; k += 4) a[0] += part[k * E + ec];
-    s_sum[wv][lane] = (a[0] + a[1]) + (a[2] + a[3]);
+    const int64_t stride = static_cast<int64_t>(gridDim.x) * STEP;
+    for (int64_t base = static_cast<int64_t>(blockIdx.x) * STEP + wv * RPW * RPT + sub; base - sub < p.rows;
+         base += stride) {
+        uint4 xr[RPT], zr[RPT], gr[RPT];
+#pragma unroll
+        for (int j = 0; j < RPT; ++j) {
+            const int64_t row = base + j * RPW < p.rows ? base + j * RPW : p.rows - 1;  // valid address
+            xr[j] = *reinterpret_cast<const uint4 *>(x + row * N + c0);
+            zr[j] = *reinterpret_cast<const uint4 *>(z + row * N + c0);
+            gr[j] = *reinterpret_cast<const uint4 *>(dy + row * N + c0);
+        }
+#pragma unroll
+        for (int j = 0; j < RPT; ++j) {
+            const int64_t row = base + j * RPW;
+            const bool live = row < p.rows;
+            const T *xe = reinterpret_cast<const T *>(&xr[j]), *ze = reinterpret_cast<const T *>(&zr[j]);
+            const T *ge = reinterpret_cast<const T *>(&gr[j]);
+            float xv[EPV], sq = 0.0f;
+#pragma unroll
+            for (int i = 0; i < EPV; ++i) {
+                xv[i] = io<T>::ld(xe, i);
+                sq = fmaf(xv[i], xv[i], sq);
+            }
+#pragma unroll
+            for (int off = LPR / 2; off > 0; off >>= 1) sq += __shfl_xor(sq, off, kWave);
+            const float r = rsqrtf(sq / static_cast<float>(N) + p.eps);
+            float g[EPV], dot = 0.0f;
+            alignas(16) T oz[EPV], ox[EPV];
+#pragma unroll
+            for (int i = 0; i < EPV; ++i) {
+                const float zv = io<T>::ld(ze, i), gv = io<T>::ld(ge, i);
+                xv[i] *= r;
+                const float sg = sigmoid_of<T>(zv);
+                const float sz = zv * sg;
+                g[i] = gv * w[i] * sz;
+                dot = fmaf(g[i], xv[i], dot);
+                io<T>::st(oz, i, gv * xv[i] * w[i] * (sg * (1.0f + zv * (1.0f - sg))));
+                if (live) acc[i] = fmaf(gv, xv[i] * sz, acc[i]);
+            }
+#pragma unroll
+            for (int off = LPR / 2; off > 0; off >>= 1) dot += __shfl_xor(dot, off, kWave);
+            dot /= static_cast<float>(N);
+#pragma unroll
+            for (int i = 0; i < EPV; ++i) io<T>::st(ox, i, r * (g[i] - xv[i] * dot));
+            if (live) {
+                *reinterpret_cast<uint4 *>(dz + row * N + c0) = *reinterpret_cast<const uint4 *>(oz);
+                *reinterpret_cast<uint4 *>(dx + row * N + c0) = *reinterpret_cast<const uint4 *>(ox);
+            }
+        }
+    }
+#pragma unroll
+    for (int off = LPR; off < kWave; off <<= 1)
+#pragma unroll
+        for (int i = 0; i < EPV; ++i) acc[i] += __shfl_xor(acc[i], off, kWave);
+    if (sub == 0) {
+#pragma unroll
+        for (int i = 0; i < EPV; ++i) s_acc[wv][c0 + i] = acc[i];
+    }
     __syncthreads();
-    if (wv != 0 || e >= E) return;
-    const float s = (s_sum[0][lane] + s_sum[1][lane]) + (s_sum[2][lane] + s_sum[3][lane]);
+    for (int c = threadIdx.x; c < N; c += 256)
+        p.part[static_cast<int64_t>(blockIdx.x) * N + c] = (s_acc[0][c] + s_acc[1][c]) + (s_acc[2][c] + s_acc[3][c]);
+}
+
+// out[e] = sum over k < nparts of part[k * E + e], e < E, in a fixed order
+// (deterministic), 64 consecutive e a workgroup of sixteen waves.  Written in
+// TO.  With W > 0, elements e = j * D + d of [W + 1][D] partials go to a
+// [D][W] weight (j < W) and a [D] bias (j == W).  A chain of waits: the norm
+// weight's 1024 partial rows of 64 are one workgroup, which took 20.0 us with
+// four waves of four requests each and takes 5.2 with sixteen of eight; the
+// 256 rows of 5120 of a convolution went from 6.8 to 4.0 us.
+template <typename TO>
+__global__ __launch_bounds__(1024) void partial_reduce_kernel(const float *part, int64_t nparts, int64_t E,
+                                                              void *out, void *out_bias, int D, int W)
+{
+    __shared__ float s_sum[16][64];
+    const int64_t e = static_cast<int64_t>(blockIdx.x) * 64 + (threadIdx.x & 63);
+    const float s = sum_parts<16, 8>(part, nparts, E, e < E ? e : E - 1, s_sum);
+    if (threadIdx.x >= 64 || e >= E) return;
     if (W == 0) {
         io<TO>::st(static_cast<TO *>(out), e, s);
         return;
@@ -234,7 +328,7 @@ hipError_t conv_bwd_w(const ConvBwdParams &p, hipStream_t s)
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     const int64_t E = static_cast<int64_t>(W + 1) * p.D;
-    hipLaunchKernelGGL((partial_reduce_kernel<T>), dim3(static_cast<unsigned>((E + 63) / 64)), dim3(256), 0, s,
+    hipLaunchKernelGGL((partial_reduce_kernel<T>), dim3(static_cast<unsigned>((E + 63) / 64)), dim3(1024), 0, s,
                        p.part, static_cast<int64_t>(p.B) * tiles, E, p.dw, p.dbias, p.D, W);
     return hipGetLastError();
 }
@@ -258,8 +352,25 @@ template <typename T, typename TW>
 hipError_t norm_bwd_t(const NormBwdParams &p, hipStream_t s)
 {
     const int blocks = static_cast<int>(norm_bwd_blocks(p.rows));
-    // Columns per lane: N <= 64, 128 or 256.
-    if (p.N <= 64)
+    constexpr int EPV = 16 / static_cast<int>(sizeof(T));
+    const int lpr = p.N % EPV == 0 ? p.N / EPV : 0;
+    const uintptr_t odd = (reinterpret_cast<uintptr_t>(p.x) | reinterpret_cast<uintptr_t>(p.z) |
+                           reinterpret_cast<uintptr_t>(p.dy) | reinterpret_cast<uintptr_t>(p.dx) |
+                           reinterpret_cast<uintptr_t>(p.dz)) % 16;
+    const auto vec = [&](auto tag) {
+        hipLaunchKernelGGL((gated_rmsnorm_bwd_vec_kernel<T, TW, decltype(tag)::value>), dim3(blocks), dim3(256), 0, s,
+                           p);
+    };
+    // Whole-piece rows; otherwise by columns per lane: N <= 64, 128 or 256.
+    if (odd == 0 && lpr == 8)
+        vec(std::integral_constant<int, 8>{});
+    else if (odd == 0 && lpr == 16)
+        vec(std::integral_constant<int, 16>{});
+    else if (odd == 0 && lpr == 32)
+        vec(std::integral_constant<int, 32>{});
+    else if (sizeof(T) == 4 && odd == 0 && lpr == 64)
+        vec(std::integral_constant<int, sizeof(T) == 4 ? 64 : 32>{});
+    else if (p.N <= 64)
         hipLaunchKernelGGL((gated_rmsnorm_bwd_kernel<T, TW, 1>), dim3(blocks), dim3(256), 0, s, p);
     else if (p.N <= 128)
         hipLaunchKernelGGL((gated_rmsnorm_bwd_kernel<T, TW, 2>), dim3(blocks), dim3(256), 0, s, p);
@@ -267,7 +378,7 @@ hipError_t norm_bwd_t(const NormBwdParams &p, hipStream_t s)
         hipLaunchKernelGGL((gated_rmsnorm_bwd_kernel<T, TW, 4>), dim3(blocks), dim3(256), 0, s, p);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((partial_reduce_kernel<TW>), dim3((p.N + 63) / 64), dim3(256), 0, s, p.part,
+    hipLaunchKernelGGL((partial_reduce_kernel<TW>), dim3((p.N + 63) / 64), dim3(1024), 0, s, p.part,
                        static_cast<int64_t>(blocks), static_cast<int64_t>(p.N), p.dweight, nullptr, p.N, 0);
     return hipGetLastError();
 }

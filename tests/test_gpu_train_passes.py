@@ -11,6 +11,26 @@ from tests._helpers import REL_TOL, rand_inputs, rel_l2, to_device
 pytestmark = pytest.mark.gpu
 
 
+@pytest.mark.parametrize("rows", [1, 17, 5000])
+@pytest.mark.parametrize("N,dtype", [(64, torch.bfloat16), (128, torch.float16), (256, torch.bfloat16),
+                                     (256, torch.float32), (32, torch.float32), (96, torch.bfloat16)])
+def test_gated_norm_backward_row_splits(gpu_device, rows, N, dtype):
+    from qwendopamine_amd.ops import gated_rmsnorm_autograd
+
+    print(f"[case] gated norm backward rows={rows} N={N} {dtype}", flush=True)
+    gen = torch.Generator().manual_seed(rows + N)
+    x, z, dy = (torch.randn(rows, N, generator=gen).to(dtype) for _ in range(3))
+    w = (torch.randn(N, generator=gen) * 0.2 + 1).to(dtype)
+    dev = [t.to(gpu_device).requires_grad_(True) for t in (x, z, w)]
+    gated_rmsnorm_autograd(*dev, 1e-5).backward(dy.to(gpu_device))
+    xd, zd, wd = ref = [t.double().requires_grad_(True) for t in (x, z, w)]
+    y = xd * torch.rsqrt(xd.square().mean(-1, keepdim=True) + 1e-5) * wd * torch.nn.functional.silu(zd)
+    y.backward(dy.double())
+    # Every value is formed in float32 and rounded once to the tensors' type.
+    for got, want in zip(dev, ref):
+        assert rel_l2(got.grad, want.grad) <= (1e-5 if dtype == torch.float32 else 4e-3)
+
+
 @pytest.mark.parametrize("T", [1, 64, 129, 300])
 @pytest.mark.parametrize("K,V", [(64, 64), (128, 40)])
 def test_float32_scans_over_chunk_counts(gpu_device, T, K, V):
