@@ -40,6 +40,7 @@ struct GateParams {
     float *part_b;    // [nblk, H, K] partial ddt_bias (null without dt_bias)
     int64_t tokens;
     int H, K, vec_ok;
+    int ql;           // backward: log2 of the lanes per row
 };
 
 // Channels 4q .. 4q+3 of row (token, h): one thread; K <= 256 (64 quads).
@@ -64,50 +65,98 @@ __global__ __launch_bounds__(256) void gate_fwd_kernel(GateParams p)
     store4(p.y, off, c0, p.K, y);
 }
 
-// Workgroup (token block tb, head h): thread (r, q) takes channels 4q..4q+3
-// of tokens tb * 64 + r, r + 4, ...; per-channel sums over its tokens, then
-// over the four token lanes in LDS.
-template <typename TG>
+// Workgroup (token block tb, head h): the QN = 2^ql lanes that cover a row's
+// channel quads (K = 64: 16) times 256 / QN token lanes r; thread (r, q) takes
+// channels 4q..4q+3 of tokens tb * 64 + r, r + 256 / QN, ..., kGateU of them
+// requested at once.  Per-channel sums over its tokens, over the token lanes
+// of a wave by shuffles, over the waves in LDS.  HBM-bound by its bytes (g, dy,
+// dg: 8 a channel in bf16); with a fixed 64 lanes a row, three quarters of them idle at
+// K = 64, and one row requested at a time it took 39.6 us at 8192 tokens x 16
+// heads x 64 channels in bf16, now 16.4 (67 MB: 4.1 TB/s).
+// VEC: K is a multiple of 4 and every row piece is aligned to its four values.
+constexpr int kGateU = 4;
+template <typename TG, bool VEC>
 __global__ __launch_bounds__(256) void gate_bwd_kernel(GateParams p)
 {
     __shared__ float s_b[4][256];
     __shared__ float s_a[4];
     const int tb = blockIdx.x / p.H, h = blockIdx.x % p.H;
-    const int q = threadIdx.x & 63, r = threadIdx.x >> 6;
-    const int c0 = 4 * q;
-    const bool live = c0 < p.K;
+    const int qn = 1 << p.ql, step = 256 >> p.ql;
+    const int q = threadIdx.x & (qn - 1), r = threadIdx.x >> p.ql, wv = threadIdx.x >> 6;
+    const bool live = 4 * q < p.K;
+    const int c0 = live ? 4 * q : 0;
     const float a = expf(p.A_log[h]);
     float db[4] = {0.f, 0.f, 0.f, 0.f};
-    if (p.dt_bias && live) load4(p.dt_bias, static_cast<int64_t>(h) * p.K, c0, p.K, true, p.vec_ok, db);
+    if (p.dt_bias) load4(p.dt_bias, static_cast<int64_t>(h) * p.K, c0, p.K, live, 0, db);
     float sb[4] = {0.f, 0.f, 0.f, 0.f}, sa = 0.f;
-    const int64_t t_end = p.tokens < static_cast<int64_t>(tb + 1) * kGateBT ? p.tokens
-                                                                           : static_cast<int64_t>(tb + 1) * kGateBT;
-    for (int64_t t = static_cast<int64_t>(tb) * kGateBT + r; t < t_end; t += 4) {
-        if (!live) break;
-        const int64_t off = (t * p.H + h) * p.K;
-        float x[4], dy[4], dg[4];
-        load4(static_cast<const TG *>(p.g), off, c0, p.K, true, p.vec_ok, x);
-        load4(p.dy, off, c0, p.K, true, p.vec_ok, dy);
+    const int64_t t_beg = static_cast<int64_t>(tb) * kGateBT;
+    const int64_t t_end = p.tokens < t_beg + kGateBT ? p.tokens : t_beg + kGateBT;
+    const TG *g = static_cast<const TG *>(p.g);
+    using Raw = std::conditional_t<sizeof(TG) == 2, uint2, uint4>;
+    for (int64_t t = t_beg + r; t < t_end; t += kGateU * step) {
+        float x[kGateU][4], dy[kGateU][4];
+        if constexpr (VEC) {
+            // Rows past the block load its first row; their dy counts as zero.
+            Raw xr[kGateU];
+            float4 yr[kGateU];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const float xi = x[i] + db[i];
-            if (p.use_lb) {
-                const float s = sigmoid_f(a * xi);
-                dg[i] = dy[i] * (p.lower_bound * s * (1.0f - s)) * a;
-                sa = fmaf(dg[i], xi, sa);
-            } else {
-                dg[i] = -a * dy[i] * sigmoid_f(xi);
-                sa = fmaf(dy[i], -a * softplus_f(xi), sa);
+            for (int u = 0; u < kGateU; ++u) {
+                const int64_t tu = t + u * step < t_end ? t + u * step : t_beg;
+                const int64_t off = (tu * p.H + h) * p.K + c0;
+                xr[u] = *reinterpret_cast<const Raw *>(g + off);
+                yr[u] = *reinterpret_cast<const float4 *>(p.dy + off);
             }
-            sb[i] += dg[i];
+#pragma unroll
+            for (int u = 0; u < kGateU; ++u) {
+                const bool ok = live && t + u * step < t_end;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) x[u][i] = io<TG>::ld(reinterpret_cast<const TG *>(&xr[u]), i);
+                dy[u][0] = ok ? yr[u].x : 0.f;
+                dy[u][1] = ok ? yr[u].y : 0.f;
+                dy[u][2] = ok ? yr[u].z : 0.f;
+                dy[u][3] = ok ? yr[u].w : 0.f;
+            }
+        } else {
+#pragma unroll
+            for (int u = 0; u < kGateU; ++u) {
+                const bool ok = live && t + u * step < t_end;
+                const int64_t off = ((ok ? t + u * step : t_beg) * p.H + h) * p.K;
+                load4(g, off, c0, p.K, ok, 0, x[u]);
+                load4(p.dy, off, c0, p.K, ok, 0, dy[u]);
+            }
         }
-        store4(static_cast<TG *>(p.dg), off, c0, p.K, dg);  // rounded to g's dtype
+#pragma unroll
+        for (int u = 0; u < kGateU; ++u) {
+            if (!live || t + u * step >= t_end) continue;
+            float dg[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float xi = x[u][i] + db[i];
+                if (p.use_lb) {
+                    const float s = sigmoid_f(a * xi);
+                    dg[i] = dy[u][i] * (p.lower_bound * s * (1.0f - s)) * a;
+                    sa = fmaf(dg[i], xi, sa);
+                } else {
+                    dg[i] = -a * dy[u][i] * sigmoid_f(xi);
+                    sa = fmaf(dy[u][i], -a * softplus_f(xi), sa);
+                }
+                sb[i] += dg[i];
+            }
+            // Rounded to g's dtype.
+            store4(static_cast<TG *>(p.dg), ((t + u * step) * p.H + h) * p.K, c0, p.K, dg);
+        }
     }
     // Channels beyond K were never loaded (zero sums).
     sa = wave_sum(sa);
-    if ((threadIdx.x & 63) == 0) s_a[r] = sa;
+    if ((threadIdx.x & 63) == 0) s_a[wv] = sa;
+    for (int off = qn; off < kWave; off <<= 1) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) s_b[r][c0 + i] = sb[i];  // c0 + 3 <= 255
+        for (int i = 0; i < 4; ++i) sb[i] += __shfl_xor(sb[i], off, kWave);
+    }
+    if ((threadIdx.x & 63) < qn) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) s_b[wv][4 * q + i] = sb[i];  // 4 q + 3 <= 255
+    }
     __syncthreads();
     const int64_t blk = tb;
     if (threadIdx.x == 0) p.part_a[blk * p.H + h] = (s_a[0] + s_a[1]) + (s_a[2] + s_a[3]);
@@ -117,21 +166,18 @@ __global__ __launch_bounds__(256) void gate_bwd_kernel(GateParams p)
     }
 }
 
-// dA_log[h] and ddt_bias[h, c]: the blocks' partial sums added in block order.
-__global__ __launch_bounds__(256) void gate_bwd_sum_kernel(GateParams p, int nblk, float *dA_log, float *ddt_bias)
+// dA_log[h] and ddt_bias[h, c]: the blocks' partial sums in a fixed order, 64
+// elements a workgroup (the first nba workgroups take dA_log).  One thread a sum
+// over 128 blocks took 61.3 us at 16 heads x 64 channels, now 3.8.
+__global__ __launch_bounds__(1024) void gate_bwd_sum_kernel(GateParams p, int nblk, int nba, float *dA_log,
+                                                            float *ddt_bias)
 {
-    const int64_t idx = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-    const int64_t nb = static_cast<int64_t>(p.H) * p.K;
-    if (idx < p.H) {
-        float s = 0.f;
-        for (int b = 0; b < nblk; ++b) s += p.part_a[static_cast<int64_t>(b) * p.H + idx];
-        dA_log[idx] = s;
-    }
-    if (ddt_bias && idx < nb) {
-        float s = 0.f;
-        for (int b = 0; b < nblk; ++b) s += p.part_b[static_cast<int64_t>(b) * nb + idx];
-        ddt_bias[idx] = s;
-    }
+    __shared__ float s_sum[16][64];
+    const bool is_a = static_cast<int>(blockIdx.x) < nba;
+    const int64_t E = is_a ? p.H : static_cast<int64_t>(p.H) * p.K;
+    const int64_t e = static_cast<int64_t>(blockIdx.x - (is_a ? 0 : nba)) * 64 + (threadIdx.x & 63);
+    const float s = sum_parts<16, 8>(is_a ? p.part_a : p.part_b, nblk, E, e < E ? e : E - 1, s_sum);
+    if (threadIdx.x < 64 && e < E) (is_a ? dA_log : ddt_bias)[e] = s;
 }
 
 int64_t gate_blocks(int64_t tokens) { return (tokens + kGateBT - 1) / kGateBT; }
@@ -186,6 +232,7 @@ int launch_gate_bwd(const void *g, int g_dtype, const float *A_log, const float 
     p.H = H;
     p.K = K;
     p.vec_ok = (K % 4) == 0;
+    while ((4 << p.ql) < K) ++p.ql;  // K <= 256: at most 64 lanes
     const int64_t nblk = gate_blocks(tokens);
     p.part_a = static_cast<float *>(workspace);
     p.part_b = dt_bias ? reinterpret_cast<float *>(static_cast<unsigned char *>(workspace) +
@@ -193,16 +240,26 @@ int launch_gate_bwd(const void *g, int g_dtype, const float *A_log, const float 
                        : nullptr;
     if (nblk > 0) {
         const dim3 grid(static_cast<unsigned>(nblk * H));
+        const auto go = [&](auto tag) {
+            using TG = decltype(tag);
+            const uintptr_t odd = (reinterpret_cast<uintptr_t>(g) | reinterpret_cast<uintptr_t>(dg)) % (4 * sizeof(TG)) |
+                                  reinterpret_cast<uintptr_t>(dy) % 16;
+            if (p.vec_ok && odd == 0)
+                hipLaunchKernelGGL((gate_bwd_kernel<TG, true>), grid, dim3(256), 0, stream, p);
+            else
+                hipLaunchKernelGGL((gate_bwd_kernel<TG, false>), grid, dim3(256), 0, stream, p);
+        };
         switch (g_dtype) {
-        case GDN2_DTYPE_F32: hipLaunchKernelGGL(gate_bwd_kernel<float>, grid, dim3(256), 0, stream, p); break;
-        case GDN2_DTYPE_BF16: hipLaunchKernelGGL(gate_bwd_kernel<bf16_t>, grid, dim3(256), 0, stream, p); break;
-        default: hipLaunchKernelGGL(gate_bwd_kernel<f16_t>, grid, dim3(256), 0, stream, p); break;
+        case GDN2_DTYPE_F32: go(float{}); break;
+        case GDN2_DTYPE_BF16: go(bf16_t{}); break;
+        default: go(f16_t{}); break;
         }
         if (hipGetLastError() != hipSuccess) return GDN2_ERR_LAUNCH;
     }
-    const int64_t n = static_cast<int64_t>(H) * K;
-    hipLaunchKernelGGL(gate_bwd_sum_kernel, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, stream, p,
-                       static_cast<int>(nblk), dA_log, dt_bias ? ddt_bias : nullptr);
+    const int nba = (H + 63) / 64;
+    const int64_t nbb = dt_bias ? (static_cast<int64_t>(H) * K + 63) / 64 : 0;
+    hipLaunchKernelGGL(gate_bwd_sum_kernel, dim3(static_cast<unsigned>(nba + nbb)), dim3(1024), 0, stream, p,
+                       static_cast<int>(nblk), nba, dA_log, ddt_bias);
     return hipGetLastError() == hipSuccess ? GDN2_OK : GDN2_ERR_LAUNCH;
 }
 

@@ -646,8 +646,16 @@ class GatedDeltaNet2(nn.Module):
         elif fuse:
             g, b, w = self.f_proj(x), self.b_proj(x), self.w_proj(x)
         else:
-            A = self.A_log.float().exp().repeat_interleave(self.head_k_dim)
-            g = -A * F.softplus(self.f_proj(x).float() + self.dt_bias)
+            f = self.f_proj(x)
+            if torch.is_grad_enabled() and f.is_cuda and f.dtype in (torch.bfloat16, torch.float16) \
+                    and self.head_k_dim <= 256:
+                # Training in 16 bits: one pass forward and one backward over the raw
+                # projection instead of torch's chain of float32 passes (float32
+                # modules keep torch's library softplus).
+                g = ops.gate_activation(_split_heads(f, self.head_k_dim), self.A_log, self.dt_bias, None).flatten(-2)
+            else:
+                A = self.A_log.float().exp().repeat_interleave(self.head_k_dim)
+                g = -A * F.softplus(f.float() + self.dt_bias)
             if not self.fp32_decay:
                 g = g.to(x.dtype)
             b = self.b_proj(x).sigmoid()

@@ -11,6 +11,27 @@ from tests._helpers import REL_TOL, rand_inputs, rel_l2, to_device
 pytestmark = pytest.mark.gpu
 
 
+@pytest.mark.parametrize("K,tokens,H,dtype", [(64, 257, 3, torch.bfloat16), (128, 64, 2, torch.bfloat16),
+                                              (4, 700, 70, torch.float16), (252, 66, 1, torch.float32),
+                                              (63, 130, 2, torch.bfloat16)])
+def test_gate_backward_lane_splits(gpu_device, K, tokens, H, dtype):
+    from qwendopamine_amd.ops import gate_activation
+
+    print(f"[case] gate backward K={K} tokens={tokens} H={H} {dtype}", flush=True)
+    gen = torch.Generator().manual_seed(K)
+    g = torch.randn(tokens, H, K, generator=gen).to(dtype)
+    A, db = torch.randn(H, generator=gen), torch.randn(H * K, generator=gen)
+    dy = torch.randn(tokens, H, K, generator=gen)
+    dev = [t.to(gpu_device).requires_grad_(True) for t in (g, A, db)]
+    gate_activation(*dev, None).backward(dy.to(gpu_device))
+    ref = [t.double().requires_grad_(True) for t in (g, A, db)]
+    y = -ref[1].exp()[:, None] * torch.nn.functional.softplus(ref[0] + ref[2].view(H, K))
+    y.backward(dy.double())
+    # dg leaves in g's type (half an ulp of bf16: 2^-9); the sums stay float32.
+    for got, want, tol in zip(dev, ref, (1e-5 if dtype == torch.float32 else 4e-3, 1e-5, 1e-5)):
+        assert rel_l2(got.grad, want.grad) <= tol
+
+
 @pytest.mark.parametrize("rows", [1, 17, 5000])
 @pytest.mark.parametrize("N,dtype", [(64, torch.bfloat16), (128, torch.float16), (256, torch.bfloat16),
                                      (256, torch.float32), (32, torch.float32), (96, torch.bfloat16)])
