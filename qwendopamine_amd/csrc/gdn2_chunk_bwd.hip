@@ -52,6 +52,7 @@ struct BwdParams {
     float scale;
     unsigned flags;
     int vec_ok;
+    int grads_vec;  // every gradient's base is 16-byte aligned
     const void *blob, *hs, *us;  // training workspace written by the forward
     void *dhs, *dys;                    // backward scratch
 };
@@ -654,6 +655,8 @@ __global__ __launch_bounds__(512) void chunk_bwd_kside_kernel(BwdParams p, int i
     const int64_t roff = ((t0 + r) * H + h) * K;
     const int64_t cb = static_cast<int64_t>(gc) * H + h;
     const bool l2 = (p.flags & GDN2_FLAG_L2NORM_QK) != 0;
+    const bool rows_vec = K == KP && p.grads_vec;  // whole aligned 4-value pieces in dq, dk, db, dg
+    const bool vals_vec = (V % 4) == 0 && p.grads_vec;  // in dv and dw
     const Q ident = identity_q4<PK>(l);
 
     const st *hsb = static_cast<const st *>(p.hs) + cb * (KP * VP);
@@ -764,6 +767,24 @@ __global__ __launch_bounds__(512) void chunk_bwd_kside_kernel(BwdParams p, int i
             return mma2<PK>(acc, ld_q4<PK>(a0), ld_q4<PK>(a0 + BLK), ld_q4<PK>(b0), ld_q4<PK>(b0 + BLK));
         else
             return mma1<PK>(acc, ld_q4<PK>(a0), ld_q4<PK>(b0));
+    };
+
+    // Four gradient values of a row: one store where every row allows it
+    // (uniform), else store4, whose checks per lane cost more than the store.
+    auto put_row = [&](auto *base, int64_t off, int c0, int n, bool vec, const float (&x)[4]) __attribute__((always_inline)) {
+        using T = std::remove_pointer_t<decltype(base)>;
+        if (!vec) {
+            store4<T>(base, off, c0, n, x);
+        } else if constexpr (sizeof(T) == 4) {
+            *reinterpret_cast<float4 *>(base + off + c0) = make_float4(x[0], x[1], x[2], x[3]);
+        } else {
+            Raw4<T> y;
+            y.set(x);
+            *reinterpret_cast<uint2 *>(base + off + c0) = y.u;
+        }
+    };
+    auto put4 = [&](auto *base, int c0, const float (&x)[4]) __attribute__((always_inline)) {
+        put_row(base, roff, c0, K, rows_vec, x);
     };
 
     Pre pre;
@@ -964,12 +985,30 @@ __global__ __launch_bounds__(512) void chunk_bwd_kside_kernel(BwdParams p, int i
     }
 
     // ---- V-contractions over staged slices ----
-    //   aT[J] = dAqk^T tile (J, R)    lT[J] = dY U^T tile^T (J, R)    (J <= R)
-    //   aN[I] = dAqk tile (I, R)      lN[I] = dY U^T tile (I, R)      (I >= R)
+    //   aS[J] = dAqk^T tile (J, R)    lS[J] = dY U^T tile^T (J, R)    (J <= R)
+    //   aS[I + 1] = dAqk tile (I, R)  lS[I + 1] = dY U^T tile (I, R)  (I >= R)
     //   cq[j] = dQbar, ce[j] = dY S0^T, ck[j] = dKtilde (row data, channel tile hh*NKH+j)
-    f32x4 aT[4], lT[4], aN[4], lN[4], cq[NKH], ce[NKH], ck[NKH];
+    // Which value tiles a wave forms depends on its token block R.  They are
+    // instantiated per R (by_block: one scalar branch to straight-line code), so
+    // that the tiles' LDS reads are requested together; with a branch around
+    // every tile each waited for its own.  The channel tiles and the pair
+    // products stay at a run-time R: inside the same code they spill at d_k = 128
+    // (19 to 59 registers, 1.06 to 1.13 ms).  With the tail's whole-piece
+    // reads and stores: B4 T8192 H16 d128 in bf16 1079 -> 1044 us, B4 T2048
+    // H16 d64 146 -> 135 us.
+    auto by_block = [&](auto f) __attribute__((always_inline)) {
+        if (R == 0)
+            f(std::integral_constant<int, 0>{});
+        else if (R == 1)
+            f(std::integral_constant<int, 1>{});
+        else if (R == 2)
+            f(std::integral_constant<int, 2>{});
+        else
+            f(std::integral_constant<int, 3>{});
+    };
+    f32x4 aS[5], lS[5], cq[NKH], ce[NKH], ck[NKH];
 #pragma unroll
-    for (int J = 0; J < 4; ++J) aT[J] = lT[J] = aN[J] = lN[J] = zero4();
+    for (int J = 0; J < 5; ++J) aS[J] = lS[J] = zero4();
 #pragma unroll
     for (int j = 0; j < NKH; ++j) cq[j] = ce[j] = ck[j] = zero4();
     float last_acc[NLT];  // this lane's part of rowsum(dS1 * S0) for channel tiles wv + 8t
@@ -1001,8 +1040,8 @@ __global__ __launch_bounds__(512) void chunk_bwd_kside_kernel(BwdParams p, int i
                 xv[i] = y[i] * pw[a][i];
                 xw[i] = y[i] * pv[a][i];
             }
-            store4<TI>(dvp, off, c, V, xv);
-            store4<TI>(dwp, off, c, V, xw);
+            put_row(dvp, off, c, V, vals_vec, xv);
+            put_row(dwp, off, c, V, vals_vec, xw);
         }
 #pragma unroll
         for (int t = 0; t < NLT; ++t) {
@@ -1018,17 +1057,20 @@ __global__ __launch_bounds__(512) void chunk_bwd_kside_kernel(BwdParams p, int i
                 }
             }
         }
+        by_block([&](auto rc) __attribute__((always_inline)) {
+            constexpr int RB = decltype(rc)::value;
 #pragma unroll
-        for (int J = 0; J < 4; ++J) {
-            if (J <= R) {
-                aT[J] = mmav(aT[J], blkU(J, 0), blkO(R, 0));
-                lT[J] = mmav(lT[J], blkU(J, 0), blkY(R, 0));
+            for (int J = 0; J < 4; ++J) {
+                if (J <= RB) {
+                    aS[J] = mmav(aS[J], blkU(J, 0), blkO(RB, 0));
+                    lS[J] = mmav(lS[J], blkU(J, 0), blkY(RB, 0));
+                }
+                if (J >= RB) {
+                    aS[J + 1] = mmav(aS[J + 1], blkO(J, 0), blkU(RB, 0));
+                    lS[J + 1] = mmav(lS[J + 1], blkY(J, 0), blkU(RB, 0));
+                }
             }
-            if (J >= R) {
-                aN[J] = mmav(aN[J], blkO(J, 0), blkU(R, 0));
-                lN[J] = mmav(lN[J], blkY(J, 0), blkU(R, 0));
-            }
-        }
+        });
 #pragma unroll
         for (int j = 0; j < NKH; ++j) {
             const int dt = hh * NKH + j;
@@ -1061,42 +1103,14 @@ __global__ __launch_bounds__(512) void chunk_bwd_kside_kernel(BwdParams p, int i
         const float4 tr = *reinterpret_cast<const float4 *>(&sT[R][c0]);
         const float4 ea = *reinterpret_cast<const float4 *>(&sEa[R][c0]);
         const float trv[4] = {tr.x, tr.y, tr.z, tr.w}, eav[4] = {ea.x, ea.y, ea.z, ea.w};
+        float tot[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const float kt_ = kv[j][i] * invk * fexp2(trv[i] - gv[j][i]) * eav[i];
-            const float tot = row16_scan(ck[j][i] * kt_);
-            if (m == 15) sKK[R][c0 + i] = tot;
+            tot[i] = row16_scan(ck[j][i] * kt_);
             ce[j][i] = -ce[j][i];  // dEbar = -dY S0^T
         }
-    }
-
-    // ---- causal masks and signs; diagonal tiles kept for the exact path ----
-    f32x4 dAd = zero4(), dLd = zero4(), dANd = zero4(), dLNd = zero4();
-#pragma unroll
-    for (int J = 0; J < 4; ++J) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int rT = 16 * R + m, cT = 16 * J + 4 * kg + i;
-            aT[J][i] = cT <= rT ? aT[J][i] : 0.f;
-            lT[J][i] = cT < rT ? -lT[J][i] : 0.f;
-            const int rN = 16 * J + 4 * kg + i, cN = 16 * R + m;
-            aN[J][i] = cN <= rN ? aN[J][i] : 0.f;
-            lN[J][i] = cN < rN ? -lN[J][i] : 0.f;
-        }
-        if (J == R) {
-            dAd = aT[J];
-            dLd = lT[J];
-            dANd = aN[J];
-            dLNd = lN[J];
-        }
-    }
-    Q baT[4], blT[4], baN[4], blN[4];
-#pragma unroll
-    for (int J = 0; J < 4; ++J) {
-        baT[J] = pack4<PK>(aT[J]);
-        blT[J] = pack4<PK>(lT[J]);
-        baN[J] = pack4<PK>(aN[J]);
-        blN[J] = pack4<PK>(lN[J]);
+        if (m == 15) *reinterpret_cast<float4 *>(&sKK[R][c0]) = make_float4(tot[0], tot[1], tot[2], tot[3]);
     }
 
     // ---- pair products, Horner over blocks.  With P_J the product of block
@@ -1119,6 +1133,30 @@ __global__ __launch_bounds__(512) void chunk_bwd_kside_kernel(BwdParams p, int i
         acc[2] *= f.z;
         acc[3] *= f.w;
     };
+    // Causal masks (the diagonal tiles only) and signs; the diagonal tiles are
+    // kept for the exact path.
+    f32x4 dAd = zero4(), dLd = zero4(), dANd = zero4(), dLNd = zero4();
+    Q bA[5], bL[5];
+#pragma unroll
+    for (int J = 0; J < 5; ++J) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            // Row m, column 4 kg + i of tile (R, R); of its transpose in slot R + 1.
+            const int d = J == R ? m - (4 * kg + i) : (J == R + 1 ? 4 * kg + i - m : 1);
+            aS[J][i] = d >= 0 ? aS[J][i] : 0.f;
+            lS[J][i] = d > 0 ? -lS[J][i] : 0.f;
+        }
+        if (J == R) {
+            dAd = aS[J];
+            dLd = lS[J];
+        }
+        if (J == R + 1) {
+            dANd = aS[J];
+            dLNd = lS[J];
+        }
+        bA[J] = pack4<PK>(aS[J]);
+        bL[J] = pack4<PK>(lS[J]);
+    }
 #pragma unroll
     for (int j = 0; j < NKH; ++j) {
         const int dt = hh * NKH + j, c0 = 16 * dt + 4 * kg;
@@ -1127,27 +1165,27 @@ __global__ __launch_bounds__(512) void chunk_bwd_kside_kernel(BwdParams p, int i
             if (J < R) {
                 scale_by(cq[j], &sE2[J][c0]);
                 scale_by(ce[j], &sE2[J][c0]);
-                cq[j] = pmma(cq[j], sKT, J, dt, baT[J]);
-                ce[j] = pmma(ce[j], sKT, J, dt, blT[J]);
+                cq[j] = pmma(cq[j], sKT, J, dt, bA[J]);
+                ce[j] = pmma(ce[j], sKT, J, dt, bL[J]);
             }
         }
 #pragma unroll
         for (int I = 3; I > 0; --I) {  // dk: row blocks I > R
             if (I > R) {
                 scale_by(ck[j], &sE2[I][c0]);
-                ck[j] = pmma(ck[j], sQT, I, dt, baN[I]);
-                ck[j] = pmma(ck[j], sET, I, dt, blN[I]);
+                ck[j] = pmma(ck[j], sQT, I, dt, bA[I + 1]);
+                ck[j] = pmma(ck[j], sET, I, dt, bL[I + 1]);
             }
         }
         if (!wave_slow) {  // diagonal block, factor 2^(-T_R)
-            Q dA_R = baT[0], dL_R = blT[0], dN_R = baN[0], dLN_R = blN[0];
+            Q dA_R = bA[0], dL_R = bL[0], dN_R = bA[1], dLN_R = bL[1];
 #pragma unroll
             for (int J = 1; J < 4; ++J)
                 if (J == R) {
-                    dA_R = baT[J];
-                    dL_R = blT[J];
-                    dN_R = baN[J];
-                    dLN_R = blN[J];
+                    dA_R = bA[J];
+                    dL_R = bL[J];
+                    dN_R = bA[J + 1];
+                    dLN_R = bL[J + 1];
                 }
             f32x4 tq = pmma(zero4(), sKT, R, dt, dA_R);
             f32x4 te = pmma(zero4(), sKT, R, dt, dL_R);
@@ -1203,22 +1241,25 @@ __global__ __launch_bounds__(512) void chunk_bwd_kside_kernel(BwdParams p, int i
                 }
             }
         }
-        float dbv4[4];
+        // The four channels' totals are requested together and stored as one
+        // 16-byte piece.
+        float dbv4[4], dG[4], pre_s[4], tot[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const float dG = qn[i] * cq[j][i] + en[i] * ce[j][i] - kn[i] * ck[j][i];
-            const float dbv = ce[j][i] * kn[i];
-            dbv4[i] = dbv;
+            dG[i] = qn[i] * cq[j][i] + en[i] * ce[j][i] - kn[i] * ck[j][i];
+            dbv4[i] = ce[j][i] * kn[i];
             ck[j][i] = fmaf(ce[j][i], bv[j][i], ck[j][i]);  // dk += de * b
             cq[j][i] *= p.scale;                            // w.r.t. the normalised q
             pq = fmaf(qv[j][i] * invq, cq[j][i], pq);
             pk = fmaf(kn[i], ck[j][i], pk);
-            const float pre_s = row16_scan(dG);
-            const float tot = __shfl(pre_s, 16 * kg + 15, 64);
-            if (m == 0) sDG[R][c0 + i] = tot;
-            ce[j][i] = tot - pre_s + dG;  // in-block suffix sum of dG
+            pre_s[i] = row16_scan(dG[i]);
         }
-        if (row_ok) store4<TI>(static_cast<TI *>(p.db), roff, c0, K, dbv4);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) tot[i] = __shfl(pre_s[i], 16 * kg + 15, 64);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) ce[j][i] = tot[i] - pre_s[i] + dG[i];  // in-block suffix sum of dG
+        if (m == 0) *reinterpret_cast<float4 *>(&sDG[R][c0]) = make_float4(tot[0], tot[1], tot[2], tot[3]);
+        if (row_ok) put4(static_cast<TI *>(p.db), c0, dbv4);
     }
     pq += __shfl_xor(pq, 16, 64);
     pq += __shfl_xor(pq, 32, 64);
@@ -1238,15 +1279,30 @@ __global__ __launch_bounds__(512) void chunk_bwd_kside_kernel(BwdParams p, int i
 #pragma unroll
     for (int j = 0; j < NKH; ++j) {
         const int c0 = 16 * (hh * NKH + j) + 4 * kg;
-        float dg4[4], dq4[4], dk4[4];
+        float dg4[4], dq4[4], dk4[4], later[4];
+        // Sums of the whole chunk and of the later blocks, read as whole pieces.
+        {
+            const float4 a = *reinterpret_cast<const float4 *>(&sLast[c0]);
+            float4 kk[4], dd[3];
+#pragma unroll
+            for (int R2 = 0; R2 < 4; ++R2) kk[R2] = *reinterpret_cast<const float4 *>(&sKK[R2][c0]);
+#pragma unroll
+            for (int R2 = 1; R2 < 4; ++R2) dd[R2 - 1] = *reinterpret_cast<const float4 *>(&sDG[R2][c0]);
+            later[0] = a.x + kk[0].x + kk[1].x + kk[2].x + kk[3].x;
+            later[1] = a.y + kk[0].y + kk[1].y + kk[2].y + kk[3].y;
+            later[2] = a.z + kk[0].z + kk[1].z + kk[2].z + kk[3].z;
+            later[3] = a.w + kk[0].w + kk[1].w + kk[2].w + kk[3].w;
+#pragma unroll
+            for (int R2 = 1; R2 < 4; ++R2) {
+                later[0] += R2 > R ? dd[R2 - 1].x : 0.f;
+                later[1] += R2 > R ? dd[R2 - 1].y : 0.f;
+                later[2] += R2 > R ? dd[R2 - 1].z : 0.f;
+                later[3] += R2 > R ? dd[R2 - 1].w : 0.f;
+            }
+        }
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const int c = c0 + i < KP ? c0 + i : KP - 1;
-            float later = sLast[c] + sKK[0][c] + sKK[1][c] + sKK[2][c] + sKK[3][c];
-#pragma unroll
-            for (int R2 = 1; R2 < 4; ++R2)
-                if (R2 > R) later += sDG[R2][c];
-            dg4[i] = ce[j][i] + later;
+            dg4[i] = ce[j][i] + later[i];
             float dq = cq[j][i], dk = ck[j][i];
             if (l2) {
                 // d/dx of x / max(||x||, eps): (dy - y (y . dy)) / ||x|| above eps, dy / eps below.
@@ -1256,9 +1312,9 @@ __global__ __launch_bounds__(512) void chunk_bwd_kside_kernel(BwdParams p, int i
             dq4[i] = dq;
             dk4[i] = dk;
         }
-        store4<TG>(static_cast<TG *>(p.dg), roff, c0, K, dg4);
-        store4<TI>(static_cast<TI *>(p.dq), roff, c0, K, dq4);
-        store4<TI>(static_cast<TI *>(p.dk), roff, c0, K, dk4);
+        put4(static_cast<TG *>(p.dg), c0, dg4);
+        put4(static_cast<TI *>(p.dq), c0, dq4);
+        put4(static_cast<TI *>(p.dk), c0, dk4);
     }
     }
     // sRow, sT and the block tables are rewritten by the next item.  With the
@@ -1363,6 +1419,9 @@ int launch_chunk_bwd(const ChunkBwdArgs &a, int io_dtype, int g_dtype, hipStream
     p.scale = a.scale;
     p.flags = a.flags;
     p.vec_ok = (a.K % 4) == 0;
+    p.grads_vec = ((reinterpret_cast<uintptr_t>(a.dq) | reinterpret_cast<uintptr_t>(a.dk) |
+                    reinterpret_cast<uintptr_t>(a.db) | reinterpret_cast<uintptr_t>(a.dg) |
+                    reinterpret_cast<uintptr_t>(a.dv) | reinterpret_cast<uintptr_t>(a.dw)) % 16) == 0;
     const unsigned char *sv = static_cast<const unsigned char *>(a.saved);
     unsigned char *wk = static_cast<unsigned char *>(a.workspace);
     p.blob = sv;
