@@ -207,4 +207,6 @@ def ptr(t: torch.Tensor | None) -> int | None:
 
 
 def stream_handle(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    # The handle itself: a Stream object built around it for every launch costs
+    # more host time than the launch's arguments.
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if device.index is None else device.index)

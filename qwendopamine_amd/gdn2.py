@@ -469,7 +469,7 @@ class GatedDeltaNet2(nn.Module):
         batch = x.shape[0]
         W_in, sizes = self._fused_input_weight()
         y = ops.linear(x.reshape(batch, x.shape[-1]), W_in)  # [B, sum(sizes)]
-        return self._decode_fused_rows(y, x.dtype, past_key_values, recurrent_state, conv_states, want_state,
+        return self._decode_fused_rows(y, sizes, x.dtype, past_key_values, recurrent_state, conv_states, want_state,
                                        in_place, use_cache)
 
     def decode_step_from_residual(self, residual: torch.Tensor, delta: torch.Tensor, norm_weight: torch.Tensor,
@@ -491,17 +491,16 @@ class GatedDeltaNet2(nn.Module):
             return None
         W_in, sizes = self._fused_input_weight()
         y, s = ops.linear_addnorm(residual.reshape(batch, -1), delta.reshape(batch, -1), norm_weight, eps, W_in)
-        out, _, _ = self._decode_fused_rows(y, residual.dtype, cache, state, tuple(conv), True, True, True)
+        out, _, _ = self._decode_fused_rows(y, sizes, residual.dtype, cache, state, tuple(conv), True, True, True)
         return s.view_as(residual), out
 
-    def _decode_fused_rows(self, y, dt, past_key_values, recurrent_state, conv_states, want_state, in_place,
+    def _decode_fused_rows(self, y, sizes, dt, past_key_values, recurrent_state, conv_states, want_state, in_place,
                            use_cache):
         """The fused decode step from the input projections' output ``y`` [B, sum(sizes)]."""
         batch = y.shape[0]
-        _, sizes = self._fused_input_weight()
         qr, kr, vr, b, w, f0, g0 = y.split(sizes, dim=-1)
-        g, z = ops.linear_pair(f0, self.f_proj[1].weight, self.f_proj[1].bias, g0, self.g_proj[1].weight,
-                               self.g_proj[1].bias)
+        f1, g1 = self.f_proj[1], self.g_proj[1]
+        g, z = ops.linear_pair(f0, f1.weight, f1.bias, g0, g1.weight, g1.bias)
         caches = list(conv_states) if all(c is not None for c in conv_states) else None
         if caches is not None and not all(c.dtype == dt and c.is_contiguous() for c in caches):
             caches, in_place = [c.to(dt).contiguous() for c in caches], False
