@@ -15,8 +15,8 @@
 //              (y itself, or dg * x for the bounded form)
 //   ddt_bias = sum over tokens of dg
 // One workgroup per (64-token block, head) writes its partial sums of dA_log
-// and ddt_bias to a workspace; a second kernel adds the blocks in order, so
-// the result does not depend on scheduling.
+// and ddt_bias to a workspace; a second kernel adds the blocks in a fixed order,
+// so the result does not depend on scheduling.
 #include <hip/hip_runtime.h>
 
 #include "gdn2_chunk.h"
