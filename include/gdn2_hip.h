@@ -66,6 +66,10 @@ enum gdn2_status {
                                   * kernels use sigmoid(b), sigmoid(w) in fp32   *
                                   * (the module's b_proj / w_proj activations,   *
                                   * gdn2.py:864-865)                             */
+#define GDN2_FLAG_LIBRARY_MATH 128u /* gdn2_gate_fwd / gdn2_gate_bwd without     *
+                                     * LOWER_BOUND: the library's exponential    *
+                                     * and logarithm, as torch's softplus takes  *
+                                     * them, instead of the hardware's           */
 
 int gdn2_abi_version(void);
 const char *gdn2_status_string(int status);
@@ -338,7 +342,10 @@ int gdn2_argmax_rows(const void *x, int64_t x_row_stride, int io_dtype, int64_t 
  * the formula of GDN2_FLAG_GATE_IN_KERNEL.  gdn2_gate_fwd writes y (float32);
  * gdn2_gate_bwd takes dy (float32) and writes dg_raw (g_dtype), dA_log [H] and
  * ddt_bias [H*K] (float32; NULL with dt_bias NULL), the two sums over tokens
- * taken per 64-token block and then added in block order (deterministic).
+ * taken per 64-token block and then added in a fixed order (deterministic).
+ * With GDN2_FLAG_LIBRARY_MATH (not with LOWER_BOUND) y equals torch's float32
+ * -exp(A_log) * softplus(g_raw + dt_bias) bit for bit, and dg_raw before its
+ * rounding torch's gradient of it.
  * workspace: at least gdn2_gate_bwd_workspace_size() bytes.
  */
 size_t gdn2_gate_bwd_workspace_size(int64_t tokens, int H, int K, int has_dt_bias);

@@ -453,7 +453,8 @@ static int check_gate_args(const void *g_raw, int g_dtype, const float *A_log, u
                            int H, int K)
 {
     if (!valid_dtype(g_dtype) || tokens < 0 || H <= 0 || K <= 0) return GDN2_ERR_INVALID;
-    if (flags & ~GDN2_FLAG_LOWER_BOUND) return GDN2_ERR_INVALID;
+    if (flags & ~(GDN2_FLAG_LOWER_BOUND | GDN2_FLAG_LIBRARY_MATH)) return GDN2_ERR_INVALID;
+    if ((flags & GDN2_FLAG_LOWER_BOUND) && (flags & GDN2_FLAG_LIBRARY_MATH)) return GDN2_ERR_INVALID;
     if (K > 256) return GDN2_ERR_UNSUPPORTED;
     if (!A_log || (tokens > 0 && !g_raw)) return GDN2_ERR_INVALID;
     return GDN2_OK;

@@ -6,7 +6,9 @@
 //   y = -exp(A_log[h]) * softplus(x)                     (default)
 //   y = lower_bound * sigmoid(exp(A_log[h]) * x)         (GDN2_FLAG_LOWER_BOUND)
 // in fp32, the same formula the chunk and token-serial kernels apply under
-// GDN2_FLAG_GATE_IN_KERNEL (gate_activation in gdn2_common.h).
+// GDN2_FLAG_GATE_IN_KERNEL (gate_activation in gdn2_common.h).  With
+// GDN2_FLAG_LIBRARY_MATH the default form and its VJP take the library's expf and
+// log1pf in the order of torch's float32 chain: y is that chain's bit for bit.
 //
 // Backward (reference kda_gate_bwd, chunk_kda.py:3254-3292, kernel
 // :3151-3220): given dy = dL/dy,
@@ -43,8 +45,22 @@ struct GateParams {
     int ql;           // backward: log2 of the lanes per row
 };
 
+// GDN2_FLAG_LIBRARY_MATH: softplus(x) and its VJP as torch forms them (threshold
+// 20), from e = expf(x): log1p(e), and t e / (e + 1) for an upstream t.  For callers
+// that held the decay in torch's float32 before; its rms error against float64 (4096
+// tokens x 16 heads x 64 channels, raw gate N(0, 2) in bf16) is 1.2e-7 with these and
+// 2.0e-7 with the hardware exp2 / log2 forms.  log1pf alone is about 130
+// instructions, which then bound both passes: 28.3 us forward and 34.2 backward at
+// 8192 tokens x 16 heads x 64 channels in bf16, 15.0 and 16.1 without.
+__device__ __forceinline__ float softplus_of_exp(float x, float e) { return x > 20.0f ? x : log1pf(e); }
+
+__device__ __forceinline__ float softplus_vjp(float x, float e, float t)
+{
+    return x > 20.0f ? t : t * e / (e + 1.0f);
+}
+
 // Channels 4q .. 4q+3 of row (token, h): one thread; K <= 256 (64 quads).
-template <typename TG>
+template <typename TG, bool LIB>
 __global__ __launch_bounds__(256) void gate_fwd_kernel(GateParams p)
 {
     const int64_t rows = p.tokens * p.H;
@@ -61,7 +77,11 @@ __global__ __launch_bounds__(256) void gate_fwd_kernel(GateParams p)
     const float a_log = p.A_log[h];
     float y[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) y[i] = gate_activation(x[i], a_log, db[i], p.use_lb, p.lower_bound);
+    for (int i = 0; i < 4; ++i) {
+        const float xi = x[i] + db[i];
+        y[i] = LIB ? -expf(a_log) * softplus_of_exp(xi, expf(xi))
+                   : gate_activation(x[i], a_log, db[i], p.use_lb, p.lower_bound);
+    }
     store4(p.y, off, c0, p.K, y);
 }
 
@@ -72,10 +92,10 @@ __global__ __launch_bounds__(256) void gate_fwd_kernel(GateParams p)
 // of a wave by shuffles, over the waves in LDS.  HBM-bound by its bytes (g, dy,
 // dg: 8 a channel in bf16); with a fixed 64 lanes a row, three quarters of them idle at
 // K = 64, and one row requested at a time it took 39.6 us at 8192 tokens x 16
-// heads x 64 channels in bf16, now 16.4 (67 MB: 4.1 TB/s).
+// heads x 64 channels in bf16, now 16.1 (67 MB: 4.2 TB/s).
 // VEC: K is a multiple of 4 and every row piece is aligned to its four values.
 constexpr int kGateU = 4;
-template <typename TG, bool VEC>
+template <typename TG, bool VEC, bool LIB>
 __global__ __launch_bounds__(256) void gate_bwd_kernel(GateParams p)
 {
     __shared__ float s_b[4][256];
@@ -132,7 +152,11 @@ __global__ __launch_bounds__(256) void gate_bwd_kernel(GateParams p)
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const float xi = x[u][i] + db[i];
-                if (p.use_lb) {
+                if constexpr (LIB) {
+                    const float e = expf(xi);
+                    dg[i] = softplus_vjp(xi, e, -a * dy[u][i]);
+                    sa = fmaf(dy[u][i], -a * softplus_of_exp(xi, e), sa);
+                } else if (p.use_lb) {
                     const float s = sigmoid_f(a * xi);
                     dg[i] = dy[u][i] * (p.lower_bound * s * (1.0f - s)) * a;
                     sa = fmaf(dg[i], xi, sa);
@@ -208,10 +232,17 @@ int launch_gate_fwd(const void *g, int g_dtype, const float *A_log, const float 
     const int64_t threads = tokens * H * ((K + 3) / 4);
     if (threads == 0) return GDN2_OK;
     const dim3 grid(static_cast<unsigned>((threads + 255) / 256));
+    const auto go = [&](auto tag) {
+        using TG = decltype(tag);
+        if (flags & GDN2_FLAG_LIBRARY_MATH)
+            hipLaunchKernelGGL((gate_fwd_kernel<TG, true>), grid, dim3(256), 0, stream, p);
+        else
+            hipLaunchKernelGGL((gate_fwd_kernel<TG, false>), grid, dim3(256), 0, stream, p);
+    };
     switch (g_dtype) {
-    case GDN2_DTYPE_F32: hipLaunchKernelGGL(gate_fwd_kernel<float>, grid, dim3(256), 0, stream, p); break;
-    case GDN2_DTYPE_BF16: hipLaunchKernelGGL(gate_fwd_kernel<bf16_t>, grid, dim3(256), 0, stream, p); break;
-    default: hipLaunchKernelGGL(gate_fwd_kernel<f16_t>, grid, dim3(256), 0, stream, p); break;
+    case GDN2_DTYPE_F32: go(float{}); break;
+    case GDN2_DTYPE_BF16: go(bf16_t{}); break;
+    default: go(f16_t{}); break;
     }
     return hipGetLastError() == hipSuccess ? GDN2_OK : GDN2_ERR_LAUNCH;
 }
@@ -244,10 +275,15 @@ int launch_gate_bwd(const void *g, int g_dtype, const float *A_log, const float 
             using TG = decltype(tag);
             const uintptr_t odd = (reinterpret_cast<uintptr_t>(g) | reinterpret_cast<uintptr_t>(dg)) % (4 * sizeof(TG)) |
                                   reinterpret_cast<uintptr_t>(dy) % 16;
-            if (p.vec_ok && odd == 0)
-                hipLaunchKernelGGL((gate_bwd_kernel<TG, true>), grid, dim3(256), 0, stream, p);
+            const bool vec = p.vec_ok && odd == 0, lib = (flags & GDN2_FLAG_LIBRARY_MATH) != 0;
+            if (vec && lib)
+                hipLaunchKernelGGL((gate_bwd_kernel<TG, true, true>), grid, dim3(256), 0, stream, p);
+            else if (vec)
+                hipLaunchKernelGGL((gate_bwd_kernel<TG, true, false>), grid, dim3(256), 0, stream, p);
+            else if (lib)
+                hipLaunchKernelGGL((gate_bwd_kernel<TG, false, true>), grid, dim3(256), 0, stream, p);
             else
-                hipLaunchKernelGGL((gate_bwd_kernel<TG, false>), grid, dim3(256), 0, stream, p);
+                hipLaunchKernelGGL((gate_bwd_kernel<TG, false, false>), grid, dim3(256), 0, stream, p);
         };
         switch (g_dtype) {
         case GDN2_DTYPE_F32: go(float{}); break;

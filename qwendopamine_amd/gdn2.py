@@ -649,10 +649,11 @@ class GatedDeltaNet2(nn.Module):
             if torch.is_grad_enabled() and f.is_cuda and f.dtype in (torch.bfloat16, torch.float16) \
                     and self.head_k_dim <= 256:
                 # Training in 16 bits: one pass forward and one backward over the raw
-                # projection (37 us of kernels at 8192 tokens x 1024 channels) instead
-                # of torch's chain of float32 passes (about 200 us).  Float32 modules
-                # keep torch's library softplus, which is exact to fewer ulps.
-                g = ops.gate_activation(_split_heads(f, self.head_k_dim), self.A_log, self.dt_bias, None).flatten(-2)
+                # projection (67 us of kernels at 8192 tokens x 1024 channels) instead
+                # of torch's chain of float32 passes (about 200 us), with that chain's
+                # float32 values.
+                g = ops.GateFunction.apply(_split_heads(f, self.head_k_dim), self.A_log, self.dt_bias, None,
+                                           True).flatten(-2)
             else:
                 A = self.A_log.float().exp().repeat_interleave(self.head_k_dim)
                 g = -A * F.softplus(f.float() + self.dt_bias)

@@ -336,10 +336,11 @@ def fused_recurrent_gdn2(
 class GateFunction(torch.autograd.Function):
     """The decay gate on its HIP kernels with their VJP: ``gdn2_gate_fwd`` /
     ``gdn2_gate_bwd`` (reference ``kda_gate_fwd`` / ``kda_gate_bwd`` and
-    ``KDAGateFunction``, ``chunk_kda.py:3223-3340``)."""
+    ``KDAGateFunction``, ``chunk_kda.py:3223-3340``).  ``library_math`` (no lower
+    bound) takes the library's exponential and logarithm as torch's softplus does."""
 
     @staticmethod
-    def forward(ctx, g, A_log, dt_bias, lower_bound):
+    def forward(ctx, g, A_log, dt_bias, lower_bound, library_math=False):
         name = "gate_activation"
         _require_gpu(name, g, A_log, dt_bias)
         H, K = g.shape[-2], g.shape[-1]
@@ -351,6 +352,8 @@ class GateFunction(torch.autograd.Function):
             raise ValueError(f"{name}: A_log must hold {H} values and dt_bias {H * K}, got "
                              f"{a.numel()} and {None if db is None else db.numel()}")
         flags = nat.FLAG_LOWER_BOUND if lower_bound is not None else 0
+        if library_math:
+            flags |= nat.FLAG_LIBRARY_MATH
         y = torch.empty(gr.shape, dtype=torch.float32, device=g.device)
         st = nat.load().gdn2_gate_fwd(
             nat.ptr(gr), nat.dtype_code(dt), nat.ptr(a), nat.ptr(db),
@@ -381,7 +384,7 @@ class GateFunction(torch.autograd.Function):
             nat.ptr(dA), nat.ptr(ddt), tokens, H, K, ws.data_ptr(), ws.numel(), nat.stream_handle(gr.device))
         nat.check(st, "gate_activation backward")
         d_db = None if ddt is None else ddt.to(db_meta[0]).reshape(db_meta[1])
-        return dgr.to(g_dtype), dA.to(a_dtype).reshape(a_shape), d_db, None
+        return dgr.to(g_dtype), dA.to(a_dtype).reshape(a_shape), d_db, None, None
 
 
 def gate_activation(g: torch.Tensor, A_log: torch.Tensor, dt_bias: torch.Tensor | None,

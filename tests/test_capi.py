@@ -176,6 +176,8 @@ def test_gate_argument_checks(lib):
     assert lib.gdn2_gate_fwd(None, 0, fake, None, 0.0, 0, fake, 10, 3, 100, None) == nat.ERR_INVALID
     assert lib.gdn2_gate_fwd(fake, 0, None, None, 0.0, 0, fake, 10, 3, 100, None) == nat.ERR_INVALID
     assert lib.gdn2_gate_fwd(fake, 0, fake, None, 0.0, nat.FLAG_L2NORM_QK, fake, 10, 3, 100, None) == nat.ERR_INVALID
+    assert lib.gdn2_gate_fwd(fake, 0, fake, None, 0.0, nat.FLAG_LIBRARY_MATH | nat.FLAG_LOWER_BOUND, fake, 10, 3, 100,
+                             None) == nat.ERR_INVALID
     assert lib.gdn2_gate_bwd(fake, 0, fake, fake, 0.0, 0, fake, fake, fake, None, 10, 3, 100, fake, 1 << 20,
                              None) == nat.ERR_INVALID
     assert lib.gdn2_gate_bwd(fake, 0, fake, None, 0.0, 0, fake, fake, fake, None, 10, 3, 100, fake, 8,
