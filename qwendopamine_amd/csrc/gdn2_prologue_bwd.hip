@@ -25,24 +25,17 @@ namespace gdn2 {
 
 namespace {
 
-// sigmoid(x): 16-bit tensors take the hardware exp2 and reciprocal (1 ulp each in
-// fp32) that their forward took, float32 ones the library's exponential and an IEEE
-// divide.  The convolution's backward, bound by its instructions, went from 23.5 to
-// 18.8 us at 8192 tokens x 1024 channels in bf16 with them.
-template <typename T>
-__device__ __forceinline__ float sigmoid_of(float x)
-{
-    if constexpr (sizeof(T) == 2)
-        return sigmoid_f(x);
-    else
-        return 1.0f / (1.0f + expf(-x));
-}
+// sigmoid(x) with the library's exponential and an IEEE divide for every type, as
+// torch's backward takes them: the hardware exp2 and reciprocal, whose product
+// x log2(e) is rounded once, triple its rms error (4.6e-8 to 1.5e-7 for |x| <= 12).  They would take the
+// convolution's backward from 23.7 to 19.1 us at 8192 tokens x 1024 channels in bf16
+// and the norm's from 19.3 to 16.8 us at 131072 rows of 64.
+__device__ __forceinline__ float sigmoid_exact(float x) { return 1.0f / (1.0f + expf(-x)); }
 
 // silu'(x) = sigmoid(x) (1 + x (1 - sigmoid(x))), torch's formula.
-template <typename T>
 __device__ __forceinline__ float silu_grad(float x)
 {
-    const float s = sigmoid_of<T>(x);
+    const float s = sigmoid_exact(x);
     return s * (1.0f + x * (1.0f - s));
 }
 
@@ -95,7 +88,7 @@ __global__ __launch_bounds__(256) void short_conv_bwd_kernel(ConvBwdParams p)
 #pragma unroll
         for (int j = 0; j < W; ++j) acc = fmaf(wt[j], xin[r + j], acc);
         const float pre = round_to<T>(acc + bias);  // the forward's rounded conv output
-        const float g = p.silu ? round_to<T>(gin[r] * silu_grad<T>(pre)) : gin[r];
+        const float g = p.silu ? round_to<T>(gin[r] * silu_grad(pre)) : gin[r];
         dpre[r] = t0 + r < p.T ? g : 0.0f;
     }
     float dw[W], db = 0.0f;
@@ -176,7 +169,7 @@ __global__ __launch_bounds__(256) void gated_rmsnorm_bwd_kernel(NormBwdParams p)
 #pragma unroll
             for (int i = 0; i < MAXC; ++i) {
                 xn[i] = xv[j][i] * r;
-                const float sg = 1.0f / (1.0f + expf(-zv[j][i]));
+                const float sg = sigmoid_exact(zv[j][i]);
                 const float sz = zv[j][i] * sg;
                 g[i] = gv[j][i] * wv_[i] * sz;
                 dot = fmaf(g[i], xn[i], dot);
@@ -209,7 +202,7 @@ __global__ __launch_bounds__(256) void gated_rmsnorm_bwd_kernel(NormBwdParams p)
 // two, 8 to 32 in 16 bits, to 64 in 32) whole 16-byte pieces; the others stay on the kernel above.
 // HBM-bound by its bytes (x, z, dy, dx, dz: 10 a value in bf16); one 2-byte value a lane
 // left it bound by shuffles and instructions: 32.6 us at 131072 rows of 64 in
-// bf16, now 17.7 (84 MB: 4.7 TB/s).
+// bf16, now 19.3 (84 MB: 4.4 TB/s).
 template <typename T, typename TW, int LPR>
 __global__ __launch_bounds__(256) void gated_rmsnorm_bwd_vec_kernel(NormBwdParams p)
 {
@@ -261,7 +254,7 @@ __global__ __launch_bounds__(256) void gated_rmsnorm_bwd_vec_kernel(NormBwdParam
             for (int i = 0; i < EPV; ++i) {
                 const float zv = io<T>::ld(ze, i), gv = io<T>::ld(ge, i);
                 xv[i] *= r;
-                const float sg = sigmoid_of<T>(zv);
+                const float sg = sigmoid_exact(zv);
                 const float sz = zv * sg;
                 g[i] = gv * w[i] * sz;
                 dot = fmaf(g[i], xv[i], dot);

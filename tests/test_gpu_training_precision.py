@@ -62,3 +62,50 @@ def test_gate_vjp_is_as_exact_as_torch(gpu_device, K, spread):
         got, want = _rms(a, e), _rms(b, e)
         print(f"  {name}: rms {got:.3g}, torch {want:.3g}", flush=True)
         assert got <= room * want, name
+
+
+def _misrounded(x, exact):
+    return (x != exact.to(x.dtype)).sum().item()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_conv_silu_backward_is_as_exact_as_torch(gpu_device, dtype):
+    from qwendopamine_amd.ops import short_conv_autograd
+
+    print(f"[case] conv backward precision {dtype}", flush=True)
+    gen = torch.Generator().manual_seed(1)
+    x = (torch.randn(4, 2048, 1024, generator=gen) * 3).to(dtype).to(gpu_device)
+    dy = torch.randn(x.shape, generator=gen).to(dtype).to(gpu_device)
+    w = torch.zeros(1024, 1, 4, dtype=dtype, device=gpu_device)
+    w[:, 0, 3] = 1  # the convolution passes x on: dx = round(dy silu'(x))
+    hip, ref = x.clone().requires_grad_(True), x.clone().requires_grad_(True)
+    short_conv_autograd(hip, w.requires_grad_(True), None, "silu").backward(dy)
+    F.silu(ref).backward(dy)
+    s = x.double().sigmoid()
+    exact = dy.double() * s * (1 + x.double() * (1 - s))
+    got, want = _misrounded(hip.grad, exact), _misrounded(ref.grad, exact)
+    print(f"  misrounded {got}, torch {want}", flush=True)
+    # How often a value rounds to the wrong neighbour is in proportion to its float32 error; products
+    # contracted in one and not in the other move that error by up to a fifth.
+    assert got <= 1.2 * want + 10
+
+
+@pytest.mark.parametrize("N,dtype", [(64, torch.float16), (128, torch.float16), (256, torch.float16), (64, torch.bfloat16)])
+def test_gated_norm_silu_backward_is_as_exact_as_torch(gpu_device, N, dtype):
+    from qwendopamine_amd.ops import gated_rmsnorm_autograd
+
+    print(f"[case] gated norm backward precision N={N} {dtype}", flush=True)
+    gen = torch.Generator().manual_seed(N)
+    rows = 131072 * 64 // N
+    # Rows of +-1 (norm exactly 1), unit weights and gradients: dz = round(x silu'(z)).
+    x = (torch.randint(0, 2, (rows, N), generator=gen) * 2 - 1).to(dtype).to(gpu_device)
+    z = (torch.randn(rows, N, generator=gen) * 3).to(dtype).to(gpu_device).requires_grad_(True)
+    w = torch.ones(N, dtype=dtype, device=gpu_device)
+    gated_rmsnorm_autograd(x.clone().requires_grad_(True), z, w.requires_grad_(True), 0.0).backward(torch.ones_like(x))
+    s, zd = z.detach().double().sigmoid(), z.detach().double()
+    exact = x.double() * s * (1 + zd * (1 - s))
+    zf = z.detach().float()
+    s = 1 / (1 + torch.exp(-zf))
+    got, want = _misrounded(z.grad, exact), _misrounded((x.float() * (s * (1 + zf * (1 - s)))).to(dtype), exact)
+    print(f"  misrounded {got}, torch {want}", flush=True)
+    assert got <= 1.2 * want + 10  # as above
