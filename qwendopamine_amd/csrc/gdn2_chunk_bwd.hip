@@ -995,9 +995,13 @@ __global__ __launch_bounds__(512) void chunk_bwd_kside_kernel(BwdParams p, int i
     // products stay at a run-time R: inside the same code they spill at d_k = 128
     // (19 to 59 registers, 1.06 to 1.13 ms).  With the tail's whole-piece
     // reads and stores: B4 T8192 H16 d128 in bf16 1079 -> 1044 us, B4 T2048
-    // H16 d64 146 -> 135 us.
+    // H16 d64 146 -> 135 us.  At d_k > 128 the kernel spills, and four copies of
+    // that code spill the most (672 bytes a lane, 252 with one at a run-time R): B2
+    // T2048 H8 d256 in bf16, forward and backward 613 us, and 507 with one.
     auto by_block = [&](auto f) __attribute__((always_inline)) {
-        if (R == 0)
+        if constexpr (KP > 128)
+            f(R);
+        else if (R == 0)
             f(std::integral_constant<int, 0>{});
         else if (R == 1)
             f(std::integral_constant<int, 1>{});
@@ -1058,7 +1062,7 @@ __global__ __launch_bounds__(512) void chunk_bwd_kside_kernel(BwdParams p, int i
             }
         }
         by_block([&](auto rc) __attribute__((always_inline)) {
-            constexpr int RB = decltype(rc)::value;
+            const int RB = rc;
 #pragma unroll
             for (int J = 0; J < 4; ++J) {
                 if (J <= RB) {

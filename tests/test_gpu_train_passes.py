@@ -69,3 +69,23 @@ def test_float32_scans_over_chunk_counts(gpu_device, T, K, V):
     assert rel_l2(o, orc.recurrent_fwd(*vals)[0]) <= tol
     for x, ref in zip(leaves, orc.recurrent_vjp(*vals, do.double().numpy())):
         assert rel_l2(x.grad, ref) <= tol
+
+
+@pytest.mark.parametrize("K,V,T,dtype", [(256, 40, 129, torch.float16), (132, 64, 77, torch.float16),
+                                         (192, 48, 200, torch.bfloat16)])
+def test_wide_key_backward_over_token_blocks(gpu_device, K, V, T, dtype):
+    from qwendopamine_amd.ops import chunk_gdn2
+
+    print(f"[case] wide key backward K={K} V={V} T={T} {dtype}", flush=True)
+    t, r = to_device(rand_inputs(2, T, 2, K, V, seed=T + K), gpu_device, dtype)
+    names = ("q", "k", "v", "g", "b", "w")
+    leaves = [t[n].detach().requires_grad_(True) for n in names]
+    o, _ = chunk_gdn2(*leaves, use_qk_l2norm_in_kernel=True)
+    # Scaled as a training loop scales its loss in fp16: gradients of about 1e-5 would be subnormal.
+    # dg sums pair terms that cancel in exact arithmetic.  Beyond d_k = 128 their factors are one
+    # 16-bit plane (two, worth float32, up to 128), so each term keeps its rounding of 2^-9 while
+    # the sum loses most of its size: 6e-2 to 7e-2 of it is left, in every build so far.
+    do = (torch.randn(o.shape, generator=torch.Generator().manual_seed(T)) * 1024).to(dtype)
+    o.backward(do.to(gpu_device))
+    for n, x, ref in zip(names, leaves, orc.recurrent_vjp(*(r[n] for n in names), do.double().numpy())):
+        assert rel_l2(x.grad, ref) <= (1e-1 if n == "g" else REL_TOL[dtype]), n
