@@ -70,6 +70,9 @@ enum gdn2_status {
                                      * LOWER_BOUND: the library's exponential    *
                                      * and logarithm, as torch's softplus takes  *
                                      * them, instead of the hardware's           */
+#define GDN2_FLAG_SHORT_SEQS 256u /* gdn2_recurrent_fwd(_ex) with cu_seqlens: no *
+                                   * sequence has more than three tokens (helps   *
+                                   * to pick a kernel; results don't depend on it) */
 
 int gdn2_abi_version(void);
 const char *gdn2_status_string(int status);

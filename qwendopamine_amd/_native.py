@@ -31,6 +31,7 @@ FLAG_TRANSPOSE_STATE = 16
 FLAG_INPLACE_FINAL_STATE = 32
 FLAG_SIGMOID_BW = 64
 FLAG_LIBRARY_MATH = 128
+FLAG_SHORT_SEQS = 256
 
 OK = 0
 ERR_INVALID = -1

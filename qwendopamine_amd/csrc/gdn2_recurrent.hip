@@ -1417,6 +1417,50 @@ static hipError_t launch_seq(const RecurrentParams &p, int N, hipStream_t stream
     return hipGetLastError();
 }
 
+// Whether sequences of several tokens run faster on recurrent_fwd_kernel.  Few
+// tokens of many heads are bound by the state's bytes and by how many rounds of
+// resident workgroups move them, not by the token chain.  recurrent_seq_kernel keeps
+// 3 workgroups of 64 columns on a CU (K <= 64; 2 up to 128), the other 2 to 8 of whole
+// rows: it wins while its grid takes half as many rounds (two thirds for two tokens).
+// bf16, both in us (rows, seq): d = 128, 256 heads x 2 tokens 14.7, 12.5; 320 16.9, 18.8;
+// 512 18.0, 23.1, x 3 22.1, 24.8, x 4 25.2, 26.3, x 8 41, 35; 640 x 2 30, 28; 1024 x 2
+// 38, 42, x 3 45, 45.  d = 64, 768 x 2 10.9, 10.4; 1024 x 2 12.9, 14.3, x 3 15.7, 15.6.
+// Beyond d_k = 128 the seq kernel is the faster one throughout (512 x 2 54, 47; x 16 237, 119).
+// A state stored for every token keeps the bytes ahead of the chain longer: from a
+// pool 320 x 4 27.4, 29.6, 384 x 6 37, 40, 512 x 8 71, 63; and wide states (512-byte rows
+// against 256-byte pieces) at any length once they fill three rounds, or exceed the
+// 256 MB cache twice over: 1024 x 16 280, 346; 512 x 16 142, 178; 768 x 8 125, 123.
+// Packed lengths are on the device: known here as GDN2_FLAG_SHORT_SEQS or as the width
+// of the slot table, else taken as long (one long sequence among short ones would
+// pay 3 us a token instead of 0.5).
+static bool whole_rows_faster(const RecurrentParams &p, int N)
+{
+    if (p.K > 128) return false;
+    const bool pooled = p.state_indices && p.ht;  // a state stored for every token
+    int64_t longest = int64_t{1} << 40;
+    if (!p.cu_seqlens)
+        longest = p.T;
+    else if (p.flags & GDN2_FLAG_SHORT_SEQS)
+        longest = p.T == 2 * static_cast<int64_t>(N) ? 2 : 3;
+    else if (p.state_indices && p.idx_seq_stride > 1)
+        longest = p.idx_seq_stride;
+    const int tpr = p.V <= 16 ? 4 : p.V <= 32 ? 8 : p.V <= 64 ? 16 : 32;  // as launched below
+    const int rows = (p.K * tpr + 255) / 256;                            // state rows of a lane there
+    const int64_t heads = static_cast<int64_t>(N) * p.HV;
+    const int64_t seq_wg = heads * ((p.V + 63) / 64), row_wg = heads * ((p.V + 4 * tpr - 1) / (4 * tpr));
+    const int seq_slots = 256 * (p.K <= 64 ? 3 : 2);
+    const int row_slots = 256 * (rows <= 2 ? 8 : rows <= 4 ? 4 : rows <= 8 ? 3 : 2);
+    const int64_t seq_rounds = (seq_wg + seq_slots - 1) / seq_slots, row_rounds = (row_wg + row_slots - 1) / row_slots;
+    // Below 64 columns the seq kernel's lanes are partly idle.
+    const bool slower = longest <= 2 || p.V < 64 ? 2 * seq_rounds >= 3 * row_rounds : seq_rounds >= 2 * row_rounds;
+    if (longest <= 2) return slower;
+    const bool small = p.K <= 64 && p.V <= 64;
+    if (!pooled) return longest <= 3 && !small && slower && row_rounds <= 2;
+    if (slower && (longest <= 3 || (!small && longest <= (p.K <= 64 ? 4 : 6) && row_rounds <= 2))) return true;
+    return p.K > 64 && p.V >= 128 && longest <= 64 &&
+           (seq_wg > 3 * seq_slots || (seq_wg >= 2 * seq_slots && seq_wg * longest >= 32 * seq_slots));
+}
+
 template <typename TI, typename TG>
 static hipError_t launch_tpr(const RecurrentParams &p, int N, hipStream_t stream)
 {
@@ -1435,14 +1479,9 @@ static hipError_t launch_tpr(const RecurrentParams &p, int N, hipStream_t stream
         return hipGetLastError();
     }
     // Sequences of several tokens (two on average when packed; their lengths
-    // are on the device).  Two or three tokens of very many heads are bound by
-    // the state's bytes, which the whole-row accesses of recurrent_fwd_kernel
-    // move faster: 64 x 2 tokens of 16 heads (d = 128) 37.5 us there, 42.0 us
-    // here; 1 x 2 tokens 11.9 and 6.0 us, 64 x 4 tokens from a pool 77.9 and 78.0,
-    // 64 x 16 tokens 137 and 100.
-    const int64_t heads = static_cast<int64_t>(N) * p.HV;
+    // are on the device).
     const bool several = p.T > 1 && (!p.cu_seqlens || p.T >= 2 * static_cast<int64_t>(N));
-    if (!trans && several && !(!p.cu_seqlens && p.T < 4 && heads >= 512)) {
+    if (!trans && several && !whole_rows_faster(p, N)) {
         if (p.K <= 64) return launch_seq<TI, TG, 64>(p, N, stream);
         if (p.K <= 128) return launch_seq<TI, TG, 128>(p, N, stream);
         return launch_seq<TI, TG, 256>(p, N, stream);

@@ -275,6 +275,9 @@ def fused_recurrent_gdn2_fwd(
         flags |= nat.FLAG_INPLACE_FINAL_STATE
     if bw_logits:
         flags |= nat.FLAG_SIGMOID_BW
+    # Batches of two or three tokens a sequence may take another kernel.
+    if cu_host is not None and 2 * N <= T <= 3 * N and T > 0 and int(cu_host.diff().max()) <= 3:
+        flags |= nat.FLAG_SHORT_SEQS
     lib = nat.load()
     st = lib.gdn2_recurrent_fwd_ex(
         nat.ptr(q), nat.ptr(k), nat.ptr(v), nat.ptr(g), nat.ptr(b), nat.ptr(w),

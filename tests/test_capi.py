@@ -82,6 +82,10 @@ def test_invalid_arguments_rejected_before_launch(lib):
     st = lib.gdn2_recurrent_fwd(None, None, None, None, None, None, 0, 0, None, None, None, None,
                                 None, 0.0, None, 1, 1, 1, 1, 1, 16, 16, 1.0, nat.FLAG_GATE_IN_KERNEL, None)
     assert st == nat.ERR_INVALID
+    # the hint on packed lengths without packed sequences
+    st = lib.gdn2_recurrent_fwd(None, None, None, None, None, None, 0, 0, None, None, None, None,
+                                None, 0.0, None, 1, 1, 1, 1, 1, 16, 16, 1.0, nat.FLAG_SHORT_SEQS, None)
+    assert st == nat.ERR_INVALID
     # non-null tensors required when there are tokens
     st = lib.gdn2_chunk_fwd(None, None, None, None, None, None, 1, 0, None, None, None, None, None,
                             0.0, None, None, 1, 1, 8, 1, 16, 16, 1.0, 0, None, 0, None)
