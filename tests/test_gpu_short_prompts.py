@@ -13,20 +13,35 @@ from tests._helpers import REL_TOL, rand_inputs, rel_l2, to_device
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("B,T,H,HV,K,V,dtype,decay", [
-    (1, 2, 2, 2, 128, 128, torch.bfloat16, "paper"),
-    (2, 16, 3, 3, 64, 64, torch.float32, "paper"),
-    (1, 17, 2, 4, 128, 128, torch.float32, "unit"),
-    (2, 33, 1, 1, 65, 20, torch.float32, "paper"),
-    (1, 9, 2, 2, 200, 36, torch.float32, "unit"),
-    (1, 64, 2, 2, 256, 128, torch.bfloat16, "paper"),
-    (8, 31, 8, 8, 16, 48, torch.float16, "paper"),      # 64 heads of 48 columns: 32-column workgroups
-    (16, 18, 16, 16, 128, 132, torch.bfloat16, "unit"),  # 256 heads: 64-column workgroups
-    (2, 40, 2, 2, 128, 64, torch.float32, "sheer"),
+def _columns(heads, K, V):
+    """16-column groups of a workgroup, as the launch picks them: the most that leave 256 workgroups."""
+    for nc in (4, 2):
+        if heads * -(-V // (16 * nc)) >= 256:
+            return nc
+    return 2 if K > 128 else 1
+
+
+@pytest.mark.parametrize("B,T,H,HV,K,V,dtype,decay,nc", [
+    (1, 2, 2, 2, 128, 128, torch.bfloat16, "paper", 1),
+    (2, 16, 3, 3, 64, 64, torch.float32, "paper", 1),
+    (1, 17, 2, 4, 128, 128, torch.float32, "unit", 1),
+    (2, 33, 1, 1, 65, 20, torch.float32, "paper", 1),
+    (1, 9, 2, 2, 200, 36, torch.float32, "unit", 2),
+    (1, 64, 2, 2, 256, 128, torch.bfloat16, "paper", 2),
+    (8, 31, 8, 8, 16, 48, torch.float16, "paper", 1),
+    (4, 19, 16, 16, 128, 128, torch.float32, "paper", 2),
+    (4, 17, 16, 16, 128, 100, torch.bfloat16, "unit", 2),
+    (8, 16, 16, 16, 64, 64, torch.float32, "paper", 2),
+    (8, 18, 8, 16, 40, 52, torch.bfloat16, "paper", 2),
+    (16, 18, 16, 16, 128, 132, torch.bfloat16, "unit", 4),
+    (16, 17, 16, 16, 64, 64, torch.float32, "paper", 4),
+    (16, 9, 16, 16, 200, 36, torch.float32, "paper", 4),
+    (2, 40, 2, 2, 128, 64, torch.float32, "sheer", 1),
 ])
-def test_prompt_matches_oracle(gpu_device, B, T, H, HV, K, V, dtype, decay):
+def test_prompt_matches_oracle(gpu_device, B, T, H, HV, K, V, dtype, decay, nc):
     from qwendopamine_amd.ops import fused_recurrent_gdn2
 
+    assert _columns(B * HV, K, V) == nc
     print(f"[case] prompt B={B} T={T} H={H} HV={HV} K={K} V={V} {dtype} {decay}", flush=True)
     t, r = to_device(rand_inputs(B, T, H, K, V, HV=HV, seed=T + K, decay=decay), gpu_device, dtype)
     o, ht = fused_recurrent_gdn2(*(t[n] for n in ("q", "k", "v", "g", "b", "w")), initial_state=t["h0"],
