@@ -89,3 +89,43 @@ def test_wide_key_backward_over_token_blocks(gpu_device, K, V, T, dtype):
     o.backward(do.to(gpu_device))
     for n, x, ref in zip(names, leaves, orc.recurrent_vjp(*(r[n] for n in names), do.double().numpy())):
         assert rel_l2(x.grad, ref) <= (1e-1 if n == "g" else REL_TOL[dtype]), n
+
+
+def _off_by_one(x):
+    """An uninitialised tensor like ``x`` that starts one element past an aligned address."""
+    return torch.empty(x.numel() + 8, dtype=x.dtype, device=x.device)[1:1 + x.numel()].view(x.shape)
+
+
+@pytest.mark.parametrize("K,V,dtype", [(128, 128, torch.bfloat16), (64, 64, torch.float16), (64, 40, torch.float32)])
+def test_chunk_backward_into_unaligned_gradients(gpu_device, monkeypatch, K, V, dtype):
+    from qwendopamine_amd.backward import chunk_gdn2_bwd
+    from qwendopamine_amd.ops import chunk_gdn2_fwd
+
+    print(f"[case] unaligned gradients K={K} V={V} {dtype}", flush=True)
+    t, _ = to_device(rand_inputs(2, 130, 2, K, V, seed=K, h0_std=0), gpu_device, dtype)
+    args = [t[n] for n in ("q", "k", "v", "g", "b", "w")]
+    do = torch.randn(2, 130, 2, V, generator=torch.Generator().manual_seed(V)).to(gpu_device, dtype)
+    saved = chunk_gdn2_fwd(*args, K ** -0.5, None, False, use_qk_l2norm_in_kernel=True, save_for_bwd=True)[-1]
+    aligned = chunk_gdn2_bwd(saved, do, None, False)
+    monkeypatch.setattr(torch, "empty_like", _off_by_one)
+    shifted = chunk_gdn2_bwd(saved, do, None, False)
+    assert all(x.data_ptr() % 16 for x in shifted[:6])
+    assert all(torch.equal(x, y) for x, y in zip(aligned[:6], shifted[:6]))
+
+
+@pytest.mark.parametrize("library_math", [False, True])
+@pytest.mark.parametrize("K,dtype", [(64, torch.bfloat16), (252, torch.float32)])
+def test_gate_backward_into_unaligned_gradient(gpu_device, monkeypatch, K, dtype, library_math):
+    from qwendopamine_amd.ops import GateFunction
+
+    print(f"[case] unaligned gate gradient K={K} {dtype} library_math={library_math}", flush=True)
+    gen = torch.Generator().manual_seed(K)
+    leaves = [torch.randn(*s, generator=gen).to(d).to(gpu_device).requires_grad_(True)
+              for s, d in (((130, 3, K), dtype), ((3,), torch.float32), ((3 * K,), torch.float32))]
+    y = GateFunction.apply(*leaves, None, library_math)
+    dy = torch.randn(130, 3, K, generator=gen).to(gpu_device)
+    aligned = torch.autograd.grad(y, leaves, dy, retain_graph=True)
+    monkeypatch.setattr(torch, "empty_like", _off_by_one)
+    shifted = torch.autograd.grad(y, leaves, dy)
+    assert shifted[0].data_ptr() % 16
+    assert all(torch.equal(a, b) for a, b in zip(aligned, shifted))
