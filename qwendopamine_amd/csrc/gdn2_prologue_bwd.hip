@@ -27,9 +27,10 @@ namespace {
 
 // sigmoid(x) with the library's exponential and an IEEE divide for every type, as
 // torch's backward takes them: the hardware exp2 and reciprocal, whose product
-// x log2(e) is rounded once, triple its rms error (4.6e-8 to 1.5e-7 for |x| <= 12).  They would take the
-// convolution's backward from 23.7 to 19.1 us at 8192 tokens x 1024 channels in bf16
-// and the norm's from 19.3 to 16.8 us at 131072 rows of 64.
+// x log2(e) is rounded once, triple its rms error (4.6e-8 to 1.5e-7 for
+// |x| <= 12).  They would take the convolution's backward from 23.7 to 19.1 us at
+// 8192 tokens x 1024 channels in bf16 and the norm's from 19.3 to 16.8 us at 131072
+// rows of 64.
 __device__ __forceinline__ float sigmoid_exact(float x) { return 1.0f / (1.0f + expf(-x)); }
 
 // silu'(x) = sigmoid(x) (1 + x (1 - sigmoid(x))), torch's formula.
@@ -385,8 +386,9 @@ int64_t conv_bwd_partial_floats(int B, int T, int D, int W)
 
 int64_t norm_bwd_blocks(int64_t rows)
 {
-    // At least 16 rows (four per wave) per workgroup, at most 1024 workgroups
-    // (four per CU): one partial row per workgroup.
+    // One partial row per workgroup, at most 1024 workgroups (four per CU).  The
+    // kernel of one value a lane takes 16 rows a workgroup, the 16-byte one 8 to 64: at
+    // few rows some of its workgroups find none and write a zero partial row.
     const int64_t b = (rows + 15) / 16;
     return b < 1 ? 1 : (b > 1024 ? 1024 : b);
 }

@@ -649,7 +649,7 @@ class GatedDeltaNet2(nn.Module):
             if torch.is_grad_enabled() and f.is_cuda and f.dtype in (torch.bfloat16, torch.float16) \
                     and self.head_k_dim <= 256:
                 # Training in 16 bits: one pass forward and one backward over the raw
-                # projection (67 us of kernels at 8192 tokens x 1024 channels) instead
+                # projection (66 us of kernels at 8192 tokens x 1024 channels) instead
                 # of torch's chain of float32 passes (about 200 us), with that chain's
                 # float32 values.
                 g = ops.GateFunction.apply(_split_heads(f, self.head_k_dim), self.A_log, self.dt_bias, None,
